@@ -272,7 +272,7 @@ int linear_fwd(const void* X, const void* W, const void* b, void* Y, int M, int 
     d.M = M; d.N = N; d.C = Y; d.C2 = Y; d.Msplit = M; d.ldc = N;
     if (b && dtype == GN_BF16 && K > 0) {
         d.cbias = (const bf16_t*)b;
-        if (gemm_dma_applicable(d)) return gemm_run(d, 0, 1, dtype, dtype, s);
+        if (gemm_dma_applicable(d, 0, 1)) return gemm_run(d, 0, 1, dtype, dtype, s);
         d.cbias = nullptr;
     }
     if (b || K == 0) {

@@ -13,7 +13,12 @@
 // Blocks are remapped so each XCD (8 per MI355X, round-robin dispatch) owns a contiguous
 // range of tiles, grouped 8 tile-rows high for L2 reuse.
 //
-// fp32 path (and bf16 shapes that are not multiples of 8): a 64x64 SIMT tile kernel.
+// It takes every bf16 shape that the LDS-DMA core (gn_gemm_dma_core.h) does not: sizes or
+// leading dimensions that are not multiples of 8, unaligned operands.  Measured on an LM head
+// with an odd vocabulary (2001 tokens, 768 -> 31997, forward and both gradients, cross-entropy
+// and norms): 11.4 ms with the scalar-FMA tiles these sizes took before, 1.00 ms here.
+//
+// fp32 path: a 64x64 SIMT tile kernel.
 #include <algorithm>
 
 #include "gn_common.h"
@@ -34,22 +39,46 @@ constexpr int TILE_ELEMS = 128 * LDS_PITCH;
 // one chunk) and the transposed stores (rows 8 apart) both spread over all 8 chunk slots.
 __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 
+// 16 bytes from an address of any alignment (one dwordx4: global memory takes unaligned
+// accesses on this target)
+__device__ __forceinline__ uint4 ld16u(const bf16_t* p) {
+    uint4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+
+// the first n (< 8) of 8 elements, the rest zero
+__device__ __forceinline__ uint4 ld_head(const bf16_t* p, int n) {
+    uint32_t w[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const uint32_t lo = 2 * d < n ? (uint32_t)p[2 * d] : 0u;
+        const uint32_t hi = 2 * d + 1 < n ? (uint32_t)p[2 * d + 1] : 0u;
+        w[d] = lo | (hi << 16);
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 // Load one 128-row x 64-k operand tile into registers (4 x 16 bytes per thread).
 //   KCONTIG: element (r, k) at P[r * ld + k]    (r = row of the tile: m for A, n for B)
 //   else   : element (r, k) at P[k * ld + r]
+// Any size, leading dimension and alignment: chunks that cross the last row or k are read
+// element by element and filled with zeros.
 template <bool KCONTIG>
 __device__ __forceinline__ void load_tile(const bf16_t* __restrict__ P, int ld, int r0,
                                           int rlim, int k0, int klim, uint4 (&reg)[4]) {
     const int t = threadIdx.x;
+    // a tile inside the operand (uniform): no bounds to look at
+    const bool inside = r0 + 128 <= rlim && k0 + BK <= klim;
     if (KCONTIG) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int c = t + 256 * i;
             const int r = r0 + (c >> 3), k = k0 + (c & 7) * 8;
-            if (r < rlim && k < klim)
-                reg[i] = *reinterpret_cast<const uint4*>(P + (size_t)r * ld + k);
-            else
-                reg[i] = make_uint4(0, 0, 0, 0);
+            const bf16_t* p = P + (size_t)r * ld + k;
+            if (inside || (r < rlim && k + 8 <= klim)) reg[i] = ld16u(p);
+            else if (r < rlim && k < klim) reg[i] = ld_head(p, klim - k);
+            else reg[i] = make_uint4(0, 0, 0, 0);
         }
     } else {
         const int rc = t & 15, kg = t >> 4;  // 16 column chunks of 8, 16 groups of 4 k-rows
@@ -57,10 +86,10 @@ __device__ __forceinline__ void load_tile(const bf16_t* __restrict__ P, int ld, 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int k = k0 + kg * 4 + i;
-            if (r < rlim && k < klim)
-                reg[i] = *reinterpret_cast<const uint4*>(P + (size_t)k * ld + r);
-            else
-                reg[i] = make_uint4(0, 0, 0, 0);
+            const bf16_t* p = P + (size_t)k * ld + r;
+            if (inside || (k < klim && r + 8 <= rlim)) reg[i] = ld16u(p);
+            else if (k < klim && r < rlim) reg[i] = ld_head(p, rlim - r);
+            else reg[i] = make_uint4(0, 0, 0, 0);
         }
     }
 }
@@ -194,7 +223,7 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_mfma(GemmDesc g) {
             gemm_store_tile<CT, EPI>(g, m0 + wm * 64 + i * 32, n0 + wn * 64 + j * 32, acc[i][j]);
 }
 
-// ---- SIMT fallback: 64x64 tile, BK 16, 4x4 outputs per thread (any shape, f32 or bf16) ----
+// ---- SIMT fallback: 64x64 tile, BK 16, 4x4 outputs per thread (fp32, any shape) ----
 template <typename TI, typename CT, bool TA, bool TB, int EPI>
 __global__ __launch_bounds__(256) void gemm_simt(GemmDesc g) {
     __shared__ float sA[16][64 + 4];
@@ -549,35 +578,23 @@ int launch_simt(const GemmDesc& g, int ta, int tb, hipStream_t s) {
     return GN_OK;
 }
 
-bool mfma_applicable(const GemmDesc& g) {
-    if (g.M % 8 || g.N % 8) return false;
-    for (int s = 0; s < g.nseg; ++s)
-        if (g.Ks[s] % 8 || !al16(g.A[s]) || !al16(g.B[s]) || g.lda[s] % 8 || g.ldb[s] % 8) return false;
-    return true;
-}
-
 }  // namespace
 
 int gemm_run(const GemmDesc& d, int transA, int transB, int dtype, int c_dtype, hipStream_t s) {
     if (d.M == 0 || d.N == 0) return GN_OK;
-    if (d.bias && !(dtype == GN_BF16 && c_dtype == GN_F32 && d.epi == 0 && gemm_dma_applicable(d))) {
+    if (d.bias && !(dtype == GN_BF16 && c_dtype == GN_F32 && d.epi == 0 && gemm_dma_applicable(d, transA, transB))) {
         set_error("gemm: fused row sums need the LDS-DMA core (bf16 operands, fp32 C)");
         return GN_E_INVALID;
     }
-    if (d.cbias && !(dtype == GN_BF16 && d.epi == 0 && gemm_dma_applicable(d))) {
+    if (d.cbias && !(dtype == GN_BF16 && d.epi == 0 && gemm_dma_applicable(d, transA, transB))) {
         set_error("gemm: the fused column bias needs the LDS-DMA core (bf16 operands)");
         return GN_E_INVALID;
     }
     if (dtype == GN_BF16) {
-        if (gemm_dma_applicable(d)) return gemm_dma_launch(d, transA, transB, c_dtype, s);
-        if (mfma_applicable(d)) {
-            if (d.epi == 1) return launch_mfma<bf16_t, 1>(d, transA, transB, s);
-            if (c_dtype == GN_F32) return launch_mfma<float, 0>(d, transA, transB, s);
-            return launch_mfma<bf16_t, 0>(d, transA, transB, s);
-        }
-        if (d.epi == 1) return launch_simt<bf16_t, bf16_t, 1>(d, transA, transB, s);
-        if (c_dtype == GN_F32) return launch_simt<bf16_t, float, 0>(d, transA, transB, s);
-        return launch_simt<bf16_t, bf16_t, 0>(d, transA, transB, s);
+        if (gemm_dma_applicable(d, transA, transB)) return gemm_dma_launch(d, transA, transB, c_dtype, s);
+        if (d.epi == 1) return launch_mfma<bf16_t, 1>(d, transA, transB, s);
+        if (c_dtype == GN_F32) return launch_mfma<float, 0>(d, transA, transB, s);
+        return launch_mfma<bf16_t, 0>(d, transA, transB, s);
     }
     if (dtype == GN_F32) {
         if (d.epi == 1) {
@@ -630,7 +647,7 @@ int weight_grad(const void* dY, int ldy, const void* X, int ldx, int M, int N, i
     // end to end (12-layer decoder, one box, interleaved runs) fusing every bias beat both the
     // two-pass column sum everywhere (9.73 vs 10.01 ms per step) and fusing only GEMMs under
     // 48 us (9.94 ms): the two extra launches per bias cost more than their kernel time.
-    if (db && dtype == GN_BF16 && gemm_dma_applicable(d)) {
+    if (db && dtype == GN_BF16 && gemm_dma_applicable(d, 1, 0)) {
         d.bias = db;
         d.bias2 = db2 ? db2 : db + Msplit;
         return gemm_dma_launch(d, 1, 0, GN_F32, s);
@@ -672,7 +689,7 @@ size_t weight_grad_ws_bytes(int M, int N, int Kin, int dtype) {
             d.bias = has_bias ? alf : nullptr;
             d.bias2 = has_bias ? alf : nullptr;
             d.accumulate = acc;
-            if (!gemm_dma_applicable(d)) continue;
+            if (!gemm_dma_applicable(d, 1, 0)) continue;
             best = std::max(best, gemm_dma_part_bytes(d, 1, GN_F32));
         }
     return best;

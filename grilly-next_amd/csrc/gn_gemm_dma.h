@@ -74,7 +74,7 @@ struct VsaDesc {
 bool vsa_dma_applicable(const VsaDesc& v);
 int vsa_dma_launch(const VsaDesc& v, hipStream_t s);
 
-bool gemm_dma_applicable(const GemmDesc& g);
+bool gemm_dma_applicable(const GemmDesc& g, int transA, int transB);
 // Workspace bytes the launch of g would use for its split-K partials if part_cap were
 // unbounded (0: none).
 size_t gemm_dma_part_bytes(const GemmDesc& g, int transA, int c_dtype);

@@ -33,14 +33,23 @@ int vsa_dma_launch(const VsaDesc& v, hipStream_t s) {
     return GN_OK;
 }
 
-bool gemm_dma_applicable(const GemmDesc& g) {
+// Rows of a k-contiguous operand and k of a k-outer one may be any count: a DMA lane clamps its
+// row, or reads zeros past the last k.  A k-outer operand's rows and a k-contiguous one's k move
+// in 16-byte chunks and must be multiples of 8, and so must N (the epilogue's vector stores).
+// A K that is not a multiple of 64 needs the plain epilogue (producer-wave tiles).
+// Ragged token counts are M of the forward and input-gradient products and K of the weight
+// gradients.  Measured (us, scalar-FMA kernel that took them before -> here): FFN forward
+// 37 x 2048 -> 5632 -> 2048 1287 -> 68.6; FFN backward 1003 x 768 -> 3072 with biases 1697 ->
+// 105; LM head over 2001 tokens (768 -> 32000, forward and both gradients) 10411 -> 579.
+bool gemm_dma_applicable(const GemmDesc& g, int transA, int transB) {
     auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    if (g.M % 8 || g.N % 8 || g.M < 8 || g.N < 8) return false;
+    if (g.N % 8 || g.N < 8 || g.M < 1 || (transA && g.M % 8)) return false;
     if (g.epi == 0 && (!al(g.C) || !al(g.C2) || g.ldc % 8 || (g.cbias && !al(g.cbias)))) return false;
     if (g.epi == 1 && (!al(g.gate) || !al(g.up) || !al(g.gu) || g.ldg % 8 || g.ldgu % 8 || g.H % 8))
         return false;
     for (int s = 0; s < g.nseg; ++s) {
-        if (g.Ks[s] % BK || !al(g.A[s]) || !al(g.B[s]) || g.lda[s] % 8 || g.ldb[s] % 8) return false;
+        if (!al(g.A[s]) || !al(g.B[s]) || g.lda[s] % 8 || g.ldb[s] % 8) return false;
+        if (g.Ks[s] % BK && (g.epi == 1 || ((!transA || transB) && g.Ks[s] % 8))) return false;
     }
     return true;
 }

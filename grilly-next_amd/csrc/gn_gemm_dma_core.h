@@ -8,7 +8,8 @@
 // Block tile BM x BN x 64, 256 threads = 2 x 2 waves, wave tile (BM/2) x (BN/2) built from
 // v_mfma_f32_32x32x16_bf16 with fp32 accumulators.  Global -> LDS moves use the 16-byte
 // `global_load_lds` DMA (no VGPR staging) into two or three LDS stages, so the DMA of the
-// next tiles runs while the MFMAs of the current one execute.  Each operand stays in LDS in its global orientation:
+// next tiles runs while the MFMAs of the current one execute.  M, N and K may end anywhere
+// inside a tile that the 16-byte chunks allow (gemm_dma_applicable).  Each operand stays in LDS in its global orientation:
 //   * k-contiguous operand (rows of 64 k):   [row][k], 16-byte chunk c of row r stored at
 //     chunk c ^ swz(r); MFMA fragments are single ds_read_b128;
 //   * k-outer operand (rows of BM/BN columns): [k][col], chunk c of k-row k stored at
@@ -90,6 +91,36 @@ __device__ __forceinline__ void stage_offsets(int ld, int r0, int rlim, int wave
             const int col = min(r0 + c * 8, rlim - 8) - r0;
             vo[j] = (uint32_t)(k * ld + col) * 2u;
         }
+    }
+}
+
+// Sixteen zero bytes in device memory: what a DMA lane reads for k past the end of a product.
+__device__ const uint4 kZero16 = {0u, 0u, 0u, 0u};
+
+// Stage the last k-tile of a product whose K is not a multiple of 64 (same element map and the
+// same number of DMA instructions as stage): lanes whose k is past klim read zeros, which add
+// nothing to any output.  A k-contiguous operand needs klim % 8 == 0 (whole chunks); a k-outer
+// one takes any klim.  Reads stay inside the operands.
+template <int R, bool KC, int NW>
+__device__ __forceinline__ void stage_tail(const bf16_t* __restrict__ P, int ld, int r0, int rlim,
+                                           int k0, int klim, int dw, uint32_t s) {
+    const int lane = threadIdx.x & 63;
+    constexpr int NJ = R / (8 * NW);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int slot = 64 * (dw * NJ + j) + lane;
+        const bf16_t* src;
+        if (KC) {
+            const int r = slot >> 3, k = k0 + (((slot & 7) ^ swz(r)) * 8);
+            src = k < klim ? P + (size_t)min(r0 + r, rlim - 1) * ld + k
+                           : reinterpret_cast<const bf16_t*>(&kZero16);
+        } else {
+            constexpr int CPR = R / 8;
+            const int kr = slot / CPR, c = (slot % CPR) ^ fko(kr), k = k0 + kr;
+            src = k < klim ? P + (size_t)k * ld + min(r0 + c * 8, rlim - 8)
+                           : reinterpret_cast<const bf16_t*>(&kZero16);
+        }
+        dma16(src, s + 1024u * (uint32_t)(dw * NJ + j));
     }
 }
 
@@ -476,8 +507,8 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& g) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    const int kt0 = g.Ks[0] / BK;
-    const int KTall = kt0 + (g.nseg > 1 ? g.Ks[1] / BK : 0);
+    const int kt0 = (g.Ks[0] + BK - 1) / BK;
+    const int KTall = kt0 + (g.nseg > 1 ? (g.Ks[1] + BK - 1) / BK : 0);
     // split y takes the k-tiles [y KTall / ksplit, (y + 1) KTall / ksplit)
     const int nsplit = g.ksplit < 1 ? 1 : g.ksplit;
     const int kt_lo = (int)(((int64_t)blockIdx.y * KTall) / nsplit);
@@ -639,14 +670,33 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& g) {
     auto dma_all = [&](int tl, int buf) {
         static_for<ND>([&](auto D_) { dma_one(D_, tl, buf); });
     };
+    // The whole DMA of a tile.  With producer waves a segment's K may end inside its last tile
+    // (a ragged token count is the K of every weight gradient): that tile's DMA fills the rest
+    // with zeros.  The self-issuing kernels spread a tile's DMA over their MFMAs and take whole
+    // k-tiles only (gemm_dma_applicable, choose_tile).
+    auto dma_tile = [&](int tl, int buf) {
+        if constexpr (!SELF_DMA) {
+            const int tt = kt_lo + tl;
+            const bool s1 = tt >= kt0;
+            const int k0 = (s1 ? tt - kt0 : tt) * BK, klim = s1 ? g.Ks[1] : g.Ks[0];
+            if (k0 + BK > klim) {
+                const uint32_t base = lds0 + (uint32_t)(buf * STAGE_B);
+                stage_tail<BM, !TA, NW>(s1 ? A1 : A0, s1 ? lda1 : lda0, m0, g.M, k0, klim, dw, base);
+                stage_tail<BN, TB, NW>(s1 ? B1 : B0, s1 ? ldb1 : ldb0, n0, g.N, k0, klim, dw,
+                                       base + A_ELEMS * 2);
+                return;
+            }
+        }
+        dma_all(tl, buf);
+    };
     auto prologue_dma = [&]() {  // tiles 0 .. STAGES-1, then wait for tile 0
         set_offsets(kt_lo >= kt0 ? 1 : 0);
-        dma_all(0, 0);
+        dma_tile(0, 0);
         offsets_for(min(1, last));
-        dma_all(min(1, last), 1);
+        dma_tile(min(1, last), 1);
         if constexpr (STAGES == 3) {
             offsets_for(min(2, last));
-            dma_all(min(2, last), 2);
+            dma_tile(min(2, last), 2);
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * ND));
         } else {
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(ND));
@@ -666,7 +716,7 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& g) {
                 else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
                 __syncthreads();
                 offsets_for(min(t + STAGES, last));
-                dma_all(min(t + STAGES, last), t % STAGES);
+                dma_tile(min(t + STAGES, last), t % STAGES);
             }
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
             __syncthreads();
@@ -1004,6 +1054,12 @@ bool allow_lds(F* fn, size_t bytes) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
 }
 
+// 64-deep k-tiles of a product, and whether a segment ends inside its last one
+inline int k_tiles(const GemmDesc& g) {
+    return (g.Ks[0] + BK - 1) / BK + (g.nseg > 1 ? (g.Ks[1] + BK - 1) / BK : 0);
+}
+inline bool k_ragged(const GemmDesc& g) { return g.Ks[0] % BK || (g.nseg > 1 && g.Ks[1] % BK); }
+
 template <bool TA, bool TB, typename CT, int BM, int BN, int EPI>
 int launch_t(const GemmDesc& g, hipStream_t s) {
     // LDS: the operand stages, or the epilogue's per-wave fp32 strips [32][BN/2 + 4] if larger
@@ -1014,7 +1070,7 @@ int launch_t(const GemmDesc& g, hipStream_t s) {
     constexpr size_t smem3 = stage3_b > strips_b ? stage3_b : strips_b;
     constexpr bool fits3 = smem3 <= 160 * 1024;
     static_assert(smem2 <= 160 * 1024, "LDS per CU");
-    const int KT = (g.Ks[0] + (g.nseg > 1 ? g.Ks[1] : 0)) / BK;
+    const int KT = k_tiles(g);
     // the bias-summing variant exists for weight gradients only (fp32 C, plain epilogue)
     constexpr bool CAN_BIAS = EPI == 0 && sizeof(CT) == 4;
     const bool bias = CAN_BIAS && g.bias;
@@ -1082,7 +1138,7 @@ inline double tile_cost(const GemmDesc& g, bool ta, size_t c_bytes, int epi, int
     static constexpr double tk_kc[4] = {1.73, 0.98, 0.98, 0.57};
     static constexpr double tk_ta[4] = {1.60, 0.98, 0.90, 0.52};
     static constexpr double fixed[4] = {16.5, 6.4, 13.0, 6.4};
-    const int KT = (g.Ks[0] + (g.nseg > 1 ? g.Ks[1] : 0)) / BK;
+    const int KT = k_tiles(g);
     const int bm = kTileShapes[i][0], bn = kTileShapes[i][1];
     const long blocks = (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * ks;
     const long full = blocks / 256;
@@ -1111,7 +1167,7 @@ inline size_t part_bytes(const GemmDesc& g, int ks) {
 }
 
 inline TileChoice choose_tile(const GemmDesc& g, bool ta, size_t c_bytes, int epi) {
-    const int KT = (g.Ks[0] + (g.nseg > 1 ? g.Ks[1] : 0)) / BK;
+    const int KT = k_tiles(g);
     const bool can_split = epi == 0 && c_bytes == 4 && !g.accumulate && !g.cbias && KT >= 32;
     // GLU epilogue over a long k loop: 128 x 128 tiles.  Their two-stage variant holds two
     // blocks per CU (64 KB of LDS, 197 registers), so one block's epilogue (gate/up loads,
@@ -1123,9 +1179,11 @@ inline TileChoice choose_tile(const GemmDesc& g, bool ta, size_t c_bytes, int ep
     // eager, 8.16 -> 8.09 ms replayed, against the model's 256 x 128.  Shorter k loops keep
     // the model's choice.
     if (epi == 1 && KT >= 12) return {3, 1};
+    // 256 x 256 tiles issue their own DMA and take whole k-tiles only (gemm_body, dma_tile)
+    const int first = k_ragged(g) ? 1 : 0;
     TileChoice best{1, 1};
     double bt = tile_cost(g, ta, c_bytes, epi, 1, 1);
-    for (int i = 0; i < 4; ++i) {
+    for (int i = first; i < 4; ++i) {
         for (int ks = 1; ks <= (can_split ? 2 : 1); ++ks) {
             const double c = tile_cost(g, ta, c_bytes, epi, i, ks);
             if (c < bt) { bt = c; best = {i, ks}; }
@@ -1141,7 +1199,7 @@ inline TileChoice choose_tile(const GemmDesc& g, bool ta, size_t c_bytes, int ep
                        ((g.N + kTileShapes[best.shape][1] - 1) / kTileShapes[best.shape][1]);
     if (can_part && tiles * best.ksplit < 256) {
         double bf = tile_cost(g, ta, c_bytes, epi, best.shape, best.ksplit, true);
-        for (int i = 0; i < 4; ++i) {
+        for (int i = first; i < 4; ++i) {
             for (int ks : {3, 4, 6, 8}) {
                 if (KT / ks < 8 || part_bytes(g, ks) > g.part_cap) continue;
                 const double c = tile_cost(g, ta, c_bytes, epi, i, ks, true);
@@ -1156,7 +1214,7 @@ inline TileChoice choose_tile(const GemmDesc& g, bool ta, size_t c_bytes, int ep
     // result is bit-identical to one launch.  Measured on MI355X (fp32 C, interleaved runs):
     // 11264 x 2048 x 4096 ([dWg;dWu]) 200-204 -> 187-189 us with 8192 rows on 256 x 256;
     // 32000 x 768 x 8192 (LM-head dW) 417-423 -> 377-385 us with 21760 rows.
-    if (epi == 0 && best.ksplit == 1 && KT >= 32) {
+    if (epi == 0 && best.ksplit == 1 && KT >= 32 && first == 0) {
         const int per_round = 256 / ((g.N + 255) / 256);  // 256 x 256 row tiles per round
         double bs = 0.95 * tile_cost(g, ta, c_bytes, epi, best.shape, 1);
         TileChoice two = best;
