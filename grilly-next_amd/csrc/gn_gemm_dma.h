@@ -85,6 +85,10 @@ int gemm_dma_f32_ta0(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_f32_ta1(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s);
 int gemm_dma_glu(const GemmDesc& g, int transA, int transB, hipStream_t s);
+// Small tiles with K split over a block's waves (gn_gemm_wave.hip), for products that the core's
+// tiles would spread over too few compute units: the tile shape to run g on, or -1 (the core).
+int gemm_wave_shape(const GemmDesc& g, int transA, int transB, int c_dtype);
+int gemm_wave_launch(const GemmDesc& g, int shape, int transA, int transB, int c_dtype, hipStream_t s);
 // C (+)= sum over y < g.ksplit of the planes at g.part (index order); N % 4 == 0, C and ldc
 // 16-byte aligned.
 void launch_split_reduce(const GemmDesc& g, hipStream_t s);

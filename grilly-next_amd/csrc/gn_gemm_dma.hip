@@ -58,6 +58,7 @@ size_t gemm_dma_part_bytes(const GemmDesc& g0, int transA, int c_dtype) {
     if (g0.epi != 0 || c_dtype != GN_F32) return 0;
     GemmDesc g = g0;
     g.part_cap = ~(size_t)0;
+    if (gemm_wave_shape(g, transA, 0, c_dtype) >= 0) return 0;
     const TileChoice tc = choose_tile(g, transA != 0, sizeof(float), 0);
     return tc.ksplit > 2 ? part_bytes(g, tc.ksplit) : 0;
 }
@@ -67,6 +68,8 @@ void launch_split_reduce(const GemmDesc& g, hipStream_t s) {
 }
 
 int gemm_dma_launch(const GemmDesc& g, int transA, int transB, int c_dtype, hipStream_t s) {
+    const int wave = gemm_wave_shape(g, transA, transB, c_dtype);
+    if (wave >= 0) return gemm_wave_launch(g, wave, transA, transB, c_dtype, s);
     if (g.epi == 1) return gemm_dma_glu(g, transA, transB, s);
     if (c_dtype == GN_F32) return transA ? gemm_dma_f32_ta1(g, transB, s) : gemm_dma_f32_ta0(g, transB, s);
     return gemm_dma_bf16(g, transA, transB, s);

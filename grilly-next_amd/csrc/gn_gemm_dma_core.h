@@ -41,7 +41,14 @@ __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 // transpose read covers 4 consecutive k-rows x 64 bytes per 32 lanes; these four values
 // differ in bits 1-2 and in bits 2-3, so the read is conflict-free on a 32-bank and on a
 // 64-bank (gfx950) LDS alike (2(k & 3) left 2-way conflicts on 64 banks).
-__device__ __forceinline__ int fko(int k) { return ((k & 1) * 6) ^ (((k >> 1) & 1) * 10); }
+// Narrower tiles have fewer chunks per k-row: with 64 columns rows k and k + 2 share the same 32
+// banks and take opposite halves of them, with 32 columns four k-rows are 64 banks as they lie.
+template <int R>
+__device__ __forceinline__ int fko(int k) {
+    if constexpr (R >= 128) return ((k & 1) * 6) ^ (((k >> 1) & 1) * 10);
+    else if constexpr (R == 64) return ((k >> 1) & 1) * 4;
+    else return 0;
+}
 
 // Stage one operand tile of R rows/cols (R = BM or BN) into LDS (R*64 bf16 = R*8 chunks,
 // R/8 DMA instructions, R/32 per wave).
@@ -65,7 +72,7 @@ __device__ __forceinline__ void stage(const bf16_t* __restrict__ P, int ld, int 
         } else {
             constexpr int CPR = R / 8;  // chunks per k-row
             const int k = slot / CPR, p = slot % CPR;
-            const int c = p ^ fko(k);
+            const int c = p ^ fko<R>(k);
             const int col = min(r0 + c * 8, rlim - 8);
             src = P + (size_t)(k0 + k) * ld + col;
         }
@@ -87,7 +94,7 @@ __device__ __forceinline__ void stage_offsets(int ld, int r0, int rlim, int wave
             vo[j] = (uint32_t)(rr * ld + c * 8) * 2u;
         } else {
             constexpr int CPR = R / 8;
-            const int k = slot / CPR, c = (slot % CPR) ^ fko(k);
+            const int k = slot / CPR, c = (slot % CPR) ^ fko<R>(k);
             const int col = min(r0 + c * 8, rlim - 8) - r0;
             vo[j] = (uint32_t)(k * ld + col) * 2u;
         }
@@ -116,7 +123,7 @@ __device__ __forceinline__ void stage_tail(const bf16_t* __restrict__ P, int ld,
                            : reinterpret_cast<const bf16_t*>(&kZero16);
         } else {
             constexpr int CPR = R / 8;
-            const int kr = slot / CPR, c = (slot % CPR) ^ fko(kr), k = k0 + kr;
+            const int kr = slot / CPR, c = (slot % CPR) ^ fko<R>(kr), k = k0 + kr;
             src = k < klim ? P + (size_t)k * ld + min(r0 + c * 8, rlim - 8)
                            : reinterpret_cast<const bf16_t*>(&kZero16);
         }
@@ -145,7 +152,7 @@ __device__ __forceinline__ bf16x8_t frag(const bf16_t* s, int row0, int ks) {
         const int col = row0 + 16 * (g & 1) + 4 * (sl & 3);
         const int k = ks * 16 + 8 * (g >> 1) + (sl >> 2);
         const int c = col >> 3, within = col & 7;
-        const bf16_t* p0 = s + k * R + ((c ^ fko(k)) * 8) + within;
+        const bf16_t* p0 = s + k * R + ((c ^ fko<R>(k)) * 8) + within;
         const bf16_t* p1 = p0 + 4 * R;  // k + 4 (same swizzle: fko(k+4) == fko(k))
         s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0));
         s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p1));
@@ -166,76 +173,82 @@ __device__ __forceinline__ void glu8(const float (&v)[8], const uint32_t (&gg)[4
     }
 }
 
+// Store eight consecutive finished columns n .. n+7 of row m (in range) with 16-byte accesses.
+template <typename CT, int EPI>
+__device__ __forceinline__ void store8(const GemmDesc& g, int m, int n, float (&v)[8]) {
+    if constexpr (EPI == 0) {
+        if (g.cbias) {
+            const uint4 bw = *reinterpret_cast<const uint4*>(g.cbias + n);
+            const uint32_t w[4] = {bw.x, bw.y, bw.z, bw.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[2 * e] += __uint_as_float(w[e] << 16);
+                v[2 * e + 1] += __uint_as_float(w[e] & 0xffff0000u);
+            }
+        }
+        CT* C = reinterpret_cast<CT*>(m < g.Msplit ? g.C : g.C2);
+        const size_t idx = (size_t)(m < g.Msplit ? m : m - g.Msplit) * g.ldc + n;
+        if constexpr (sizeof(CT) == 4) {
+            float4* p = reinterpret_cast<float4*>(reinterpret_cast<float*>(C) + idx);
+            if (g.accumulate) {
+                const float4 o0 = p[0], o1 = p[1];
+                v[0] += o0.x; v[1] += o0.y; v[2] += o0.z; v[3] += o0.w;
+                v[4] += o1.x; v[5] += o1.y; v[6] += o1.z; v[7] += o1.w;
+            }
+            p[0] = make_float4(v[0], v[1], v[2], v[3]);
+            p[1] = make_float4(v[4], v[5], v[6], v[7]);
+        } else {
+            uint4* p = reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(C) + idx);
+            if (g.accumulate) {
+                const uint4 o = *p;
+                const uint32_t w[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[2 * e] += __uint_as_float(w[e] << 16);
+                    v[2 * e + 1] += __uint_as_float(w[e] & 0xffff0000u);
+                }
+            }
+            *p = make_uint4(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]),
+                            pack_bf2(v[6], v[7]));
+        }
+    } else {
+        const size_t gi = (size_t)m * g.ldg + n;
+        const uint4 gw = *reinterpret_cast<const uint4*>(g.gate + gi);
+        const uint4 uw = *reinterpret_cast<const uint4*>(g.up + gi);
+        const uint32_t gg[4] = {gw.x, gw.y, gw.z, gw.w}, uu[4] = {uw.x, uw.y, uw.z, uw.w};
+        float dg[8], du[8];
+        switch (g.glu_kind) {
+            case GN_GLU_SWIGLU_UP: glu8<GN_GLU_SWIGLU_UP>(v, gg, uu, dg, du); break;
+            case GN_GLU_SWIGLU_GATE: glu8<GN_GLU_SWIGLU_GATE>(v, gg, uu, dg, du); break;
+            case GN_GLU_GEGLU_UP: glu8<GN_GLU_GEGLU_UP>(v, gg, uu, dg, du); break;
+            case GN_GLU_GEGLU_GATE: glu8<GN_GLU_GEGLU_GATE>(v, gg, uu, dg, du); break;
+            default: glu8<GN_GLU_REGLU_UP>(v, gg, uu, dg, du); break;
+        }
+        bf16_t* o = g.gu + (size_t)m * g.ldgu + n;
+        *reinterpret_cast<uint4*>(o) = make_uint4(pack_bf2(dg[0], dg[1]), pack_bf2(dg[2], dg[3]),
+                                                  pack_bf2(dg[4], dg[5]), pack_bf2(dg[6], dg[7]));
+        *reinterpret_cast<uint4*>(o + g.H) = make_uint4(pack_bf2(du[0], du[1]), pack_bf2(du[2], du[3]),
+                                                        pack_bf2(du[4], du[5]), pack_bf2(du[6], du[7]));
+    }
+}
+
 // Write one staged 32 x WN strip (LDS, fp32, pitch WN+4) to global memory: lane l owns
 // row l/2 and WN/2 consecutive columns, moved 8 at a time with 16-byte accesses.
 template <typename CT, int EPI, int WN>
 __device__ __forceinline__ void epilogue_rows(const GemmDesc& g, const float* st, int mbase, int nbase,
                                            int lane) {
-        const int rr = lane >> 1;
-        const int m = mbase + rr;
+    const int rr = lane >> 1;
+    const int m = mbase + rr;
 #pragma unroll
-        for (int q = 0; q < WN / 16; ++q) {
-            const int c = (lane & 1) * (WN / 2) + q * 8;
-            const int n = nbase + c;
-            const float4 lo = *reinterpret_cast<const float4*>(st + rr * (WN + 4) + c);
-            const float4 hi = *reinterpret_cast<const float4*>(st + rr * (WN + 4) + c + 4);
-            float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-            if (m >= g.M || n >= g.N) continue;
-            if constexpr (EPI == 0) {
-                if (g.cbias) {
-                    const uint4 bw = *reinterpret_cast<const uint4*>(g.cbias + n);
-                    const uint32_t w[4] = {bw.x, bw.y, bw.z, bw.w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        v[2 * e] += __uint_as_float(w[e] << 16);
-                        v[2 * e + 1] += __uint_as_float(w[e] & 0xffff0000u);
-                    }
-                }
-                CT* C = reinterpret_cast<CT*>(m < g.Msplit ? g.C : g.C2);
-                const size_t idx = (size_t)(m < g.Msplit ? m : m - g.Msplit) * g.ldc + n;
-                if constexpr (sizeof(CT) == 4) {
-                    float4* p = reinterpret_cast<float4*>(reinterpret_cast<float*>(C) + idx);
-                    if (g.accumulate) {
-                        const float4 o0 = p[0], o1 = p[1];
-                        v[0] += o0.x; v[1] += o0.y; v[2] += o0.z; v[3] += o0.w;
-                        v[4] += o1.x; v[5] += o1.y; v[6] += o1.z; v[7] += o1.w;
-                    }
-                    p[0] = make_float4(v[0], v[1], v[2], v[3]);
-                    p[1] = make_float4(v[4], v[5], v[6], v[7]);
-                } else {
-                    uint4* p = reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(C) + idx);
-                    if (g.accumulate) {
-                        const uint4 o = *p;
-                        const uint32_t w[4] = {o.x, o.y, o.z, o.w};
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            v[2 * e] += __uint_as_float(w[e] << 16);
-                            v[2 * e + 1] += __uint_as_float(w[e] & 0xffff0000u);
-                        }
-                    }
-                    *p = make_uint4(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]),
-                                    pack_bf2(v[6], v[7]));
-                }
-            } else {
-                const size_t gi = (size_t)m * g.ldg + n;
-                const uint4 gw = *reinterpret_cast<const uint4*>(g.gate + gi);
-                const uint4 uw = *reinterpret_cast<const uint4*>(g.up + gi);
-                const uint32_t gg[4] = {gw.x, gw.y, gw.z, gw.w}, uu[4] = {uw.x, uw.y, uw.z, uw.w};
-                float dg[8], du[8];
-                switch (g.glu_kind) {
-                    case GN_GLU_SWIGLU_UP: glu8<GN_GLU_SWIGLU_UP>(v, gg, uu, dg, du); break;
-                    case GN_GLU_SWIGLU_GATE: glu8<GN_GLU_SWIGLU_GATE>(v, gg, uu, dg, du); break;
-                    case GN_GLU_GEGLU_UP: glu8<GN_GLU_GEGLU_UP>(v, gg, uu, dg, du); break;
-                    case GN_GLU_GEGLU_GATE: glu8<GN_GLU_GEGLU_GATE>(v, gg, uu, dg, du); break;
-                    default: glu8<GN_GLU_REGLU_UP>(v, gg, uu, dg, du); break;
-                }
-                bf16_t* o = g.gu + (size_t)m * g.ldgu + n;
-                *reinterpret_cast<uint4*>(o) = make_uint4(pack_bf2(dg[0], dg[1]), pack_bf2(dg[2], dg[3]),
-                                                          pack_bf2(dg[4], dg[5]), pack_bf2(dg[6], dg[7]));
-                *reinterpret_cast<uint4*>(o + g.H) = make_uint4(pack_bf2(du[0], du[1]), pack_bf2(du[2], du[3]),
-                                                                pack_bf2(du[4], du[5]), pack_bf2(du[6], du[7]));
-            }
-        }
+    for (int q = 0; q < WN / 16; ++q) {
+        const int c = (lane & 1) * (WN / 2) + q * 8;
+        const int n = nbase + c;
+        const float4 lo = *reinterpret_cast<const float4*>(st + rr * (WN + 4) + c);
+        const float4 hi = *reinterpret_cast<const float4*>(st + rr * (WN + 4) + c + 4);
+        float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        if (m >= g.M || n >= g.N) continue;
+        store8<CT, EPI>(g, m, n, v);
+    }
 }
 
 template <typename F, int... I>
@@ -934,7 +947,7 @@ __global__ __launch_bounds__(64 * kVsaNW, 1) void vsa_dw_dma(VsaDesc v) {
         for (int e = 0; e < 4; ++e) {
             const int b = (e + (wc >> 2)) & 3;
             const int c = 4 * wc + b;
-            *reinterpret_cast<uint4*>(sb + r * BN + ((c ^ fko(r)) * 8)) = vsa_chunk(nw, b);
+            *reinterpret_cast<uint4*>(sb + r * BN + ((c ^ fko<BN>(r)) * 8)) = vsa_chunk(nw, b);
         }
     };
     bf16x8_t fh[2][FM], fl[2][FM], fb[2][FN];

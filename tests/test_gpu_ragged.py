@@ -41,7 +41,9 @@ def gen(seed):
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 8), (8, 8, 1), (37, 264, 136), (136, 72, 1003), (257, 384, 63),
-                                   (1003, 768, 72), (768, 776, 1003), (33, 50, 77), (131, 1001, 129)])
+                                   (1003, 768, 72), (768, 776, 1003), (33, 50, 77), (131, 1001, 129),
+                                   # K split over a block's waves: rings not filled, filled, reused
+                                   (32, 32, 64), (40, 40, 320), (72, 264, 2112), (200, 136, 2600)])
 def test_gemm_any_size(gn, ta, tb, M, N, K):
     g = gen(M + N + K)
     A = guarded(g, *((K, M) if ta else (M, K)))
