@@ -258,8 +258,8 @@ __global__ __launch_bounds__(256) void fill_rows(const T* __restrict__ b, T* __r
 }
 
 // Y [M x N] = X [M x K] W^T (W [N x K]) + b, all in `dtype` (fp32 accumulation).  The bias
-// rides on the GEMM epilogue on the LDS-DMA core; other shapes start Y from the bias and
-// accumulate.
+// rides on the GEMM epilogue; bf16 shapes that the LDS-DMA core does not take start Y from the
+// bias and accumulate.
 int linear_fwd(const void* X, const void* W, const void* b, void* Y, int M, int N, int K,
                int dtype, hipStream_t s) {
     if (dtype == GN_F32 && skinny_fwd_applicable(X, W, Y, M, K))
@@ -275,7 +275,9 @@ int linear_fwd(const void* X, const void* W, const void* b, void* Y, int M, int 
         if (gemm_dma_applicable(d, 0, 1)) return gemm_run(d, 0, 1, dtype, dtype, s);
         d.cbias = nullptr;
     }
-    if (b || K == 0) {
+    if (b && dtype == GN_F32 && K > 0) {
+        d.fbias = (const float*)b;
+    } else if (b || K == 0) {
         const int64_t total = (int64_t)M * N;
         if (dtype == GN_BF16)
             fill_rows<bf16_t><<<grid_for(total, 256, 16384), 256, 0, s>>>((const bf16_t*)b, (bf16_t*)Y, total, N);

@@ -18,7 +18,7 @@
 // with an odd vocabulary (2001 tokens, 768 -> 31997, forward and both gradients, cross-entropy
 // and norms): 11.4 ms with the scalar-FMA tiles these sizes took before, 1.00 ms here.
 //
-// fp32 path: a 64x64 SIMT tile kernel.
+// fp32 path: gn_gemm_f32.hip and gn_gemm_f32mm.hip; the smallest products here (gemm_small).
 #include <algorithm>
 
 #include "gn_common.h"
@@ -221,55 +221,6 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_mfma(GemmDesc g) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
             gemm_store_tile<CT, EPI>(g, m0 + wm * 64 + i * 32, n0 + wn * 64 + j * 32, acc[i][j]);
-}
-
-// ---- SIMT fallback: 64x64 tile, BK 16, 4x4 outputs per thread (fp32, any shape) ----
-template <typename TI, typename CT, bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(256) void gemm_simt(GemmDesc g) {
-    __shared__ float sA[16][64 + 4];
-    __shared__ float sB[16][64 + 4];
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    float acc[4][4] = {};
-    for (int s = 0; s < g.nseg; ++s) {
-        const TI* A = reinterpret_cast<const TI*>(g.A[s]);
-        const TI* B = reinterpret_cast<const TI*>(g.B[s]);
-        const int Ks = g.Ks[s], lda = g.lda[s], ldb = g.ldb[s];
-        for (int k0 = 0; k0 < Ks; k0 += 16) {
-            for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-                const int kk = e / 64, mm = e % 64;
-                const int m = m0 + mm, k = k0 + kk;
-                float va = 0.f;
-                if (m < g.M && k < Ks) va = TA ? io<TI>::ld(A, (size_t)k * lda + m) : io<TI>::ld(A, (size_t)m * lda + k);
-                sA[kk][mm] = va;
-                const int n = n0 + mm;
-                float vb = 0.f;
-                if (n < g.N && k < Ks) vb = TB ? io<TI>::ld(B, (size_t)n * ldb + k) : io<TI>::ld(B, (size_t)k * ldb + n);
-                sB[kk][mm] = vb;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int kk = 0; kk < 16; ++kk) {
-                float a[4], b[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) a[i] = sA[kk][ty + 16 * i];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) b[j] = sB[kk][tx + 16 * j];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-            }
-            __syncthreads();
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int m = m0 + ty + 16 * i, n = n0 + tx + 16 * j;
-            if (m < g.M && n < g.N) gemm_store<CT, EPI>(g, m, n, acc[i][j]);
-        }
 }
 
 // ---- small products: one thread per output, the whole k loop in registers ---------------
@@ -567,23 +518,16 @@ int launch_mfma(const GemmDesc& g, int ta, int tb, hipStream_t s) {
     return launch_mfma_t<true, true, CT, EPI>(g, s);
 }
 
-template <typename TI, typename CT, int EPI>
-int launch_simt(const GemmDesc& g, int ta, int tb, hipStream_t s) {
-    dim3 grid((g.N + 63) / 64, (g.M + 63) / 64);
-    if (!ta && !tb) gemm_simt<TI, CT, false, false, EPI><<<grid, 256, 0, s>>>(g);
-    else if (!ta && tb) gemm_simt<TI, CT, false, true, EPI><<<grid, 256, 0, s>>>(g);
-    else if (ta && !tb) gemm_simt<TI, CT, true, false, EPI><<<grid, 256, 0, s>>>(g);
-    else gemm_simt<TI, CT, true, true, EPI><<<grid, 256, 0, s>>>(g);
-    GN_LAUNCH_CHECK("gn_gemm (simt)");
-    return GN_OK;
-}
-
 }  // namespace
 
 int gemm_run(const GemmDesc& d, int transA, int transB, int dtype, int c_dtype, hipStream_t s) {
     if (d.M == 0 || d.N == 0) return GN_OK;
     if (d.bias && !(dtype == GN_BF16 && c_dtype == GN_F32 && d.epi == 0 && gemm_dma_applicable(d, transA, transB))) {
         set_error("gemm: fused row sums need the LDS-DMA core (bf16 operands, fp32 C)");
+        return GN_E_INVALID;
+    }
+    if (d.fbias && !(dtype == GN_F32 && !d.accumulate)) {
+        set_error("gemm: the fp32 column bias goes with fp32 operands, overwriting C");
         return GN_E_INVALID;
     }
     if (d.cbias && !(dtype == GN_BF16 && d.epi == 0 && gemm_dma_applicable(d, transA, transB))) {
@@ -602,8 +546,8 @@ int gemm_run(const GemmDesc& d, int transA, int transB, int dtype, int c_dtype, 
             return GN_E_INVALID;
         }
         if (small_applicable(d)) return launch_small<float, float>(d, transA, transB, s);
-        if (gemm_f32_applicable(d)) return gemm_f32_launch(d, transA, transB, s);
-        return launch_simt<float, float, 0>(d, transA, transB, s);
+        if (gemm_f32_applicable(d) && !gemm_f32mm_wins(d)) return gemm_f32_launch(d, transA, transB, s);
+        return gemm_f32mm_launch(d, transA, transB, s);
     }
     set_error("gn_gemm: dtype %d not supported (f32, bf16)", dtype);
     return GN_E_INVALID;

@@ -44,6 +44,8 @@ struct GemmDesc {
     // column bias of the plain epilogue (a forward Linear's b): C[m][n] = acc + cbias[n],
     // bf16, LDS-DMA core only, no split-K; nullptr: none
     const bf16_t* cbias;
+    // the same for an fp32 product (fp32 operands and C, overwritten); nullptr: none
+    const float* fbias;
     // split-K through a workspace (plain fp32 epilogue, ksplit >= 3): split y stores its
     // partial tile at part + y*M*N (row-major, pitch N) and, with a bias, its row sums at
     // part + ksplit*M*N + y*M; split_reduce then adds the splits in index order into C and
@@ -93,10 +95,17 @@ int gemm_wave_launch(const GemmDesc& g, int shape, int transA, int transB, int c
 // 16-byte aligned.
 void launch_split_reduce(const GemmDesc& g, hipStream_t s);
 
+// fp32 operands on the fp32 matrix instruction, any size and alignment (gn_gemm_f32mm.hip);
+// _wins: it is faster than the split below for a shape that takes both
+bool gemm_f32mm_wins(const GemmDesc& g);
+int gemm_f32mm_launch(const GemmDesc& g, int transA, int transB, hipStream_t s);
+
 // fp32 operands on the bf16 MFMA pipe through a six-product three-piece split (gn_gemm_f32.hip)
 bool gemm_f32_applicable(const GemmDesc& g);
 // workspace bytes the launch would use for split-K partial planes (0: none)
 size_t gemm_f32_part_bytes(const GemmDesc& g);
+// the launch's blocks and 16-k stages per block, for a choice between the fp32 kernels
+void gemm_f32_grid(const GemmDesc& g, long& blocks, int& stages);
 int gemm_f32_launch(const GemmDesc& g, int transA, int transB, hipStream_t s);
 
 template <typename CT, int EPI>
@@ -104,6 +113,7 @@ __device__ __forceinline__ void gemm_store(const GemmDesc& g, int m, int n, floa
     if constexpr (EPI == 0) {
         CT* C = reinterpret_cast<CT*>(m < g.Msplit ? g.C : g.C2);
         const size_t idx = (size_t)(m < g.Msplit ? m : m - g.Msplit) * g.ldc + n;
+        if (g.fbias) v += g.fbias[n];
         io<CT>::st(C, idx, g.accumulate ? v + io<CT>::ld(C, idx) : v);
     } else {
         const size_t gi = (size_t)m * g.ldg + n;
@@ -177,8 +187,9 @@ int skinny_linear_bwd(const float* dY, const float* X, const float* W, float* dX
                       float* db, int M, int N, int K, bool accumulate, void* ws, size_t ws_bytes,
                       hipStream_t s, float* s_bar = nullptr, const SmHyper* sm = nullptr);
 
-// Run C (+)= sum_s op(A_s) op(B_s) described by `d`: the LDS-DMA kernel when the shape
-// allows it, else the register-staged MFMA kernel, else the SIMT kernel.
+// Run C (+)= sum_s op(A_s) op(B_s) described by `d`.  bf16: the LDS-DMA kernels when the shape
+// allows it, else the register-staged MFMA kernel.  fp32: gemm_small, the six-product split or
+// the fp32 matrix instruction, by size.
 int gemm_run(const GemmDesc& d, int transA, int transB, int dtype, int c_dtype, hipStream_t s);
 
 }  // namespace gn

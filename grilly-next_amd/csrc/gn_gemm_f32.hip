@@ -324,6 +324,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32x6(GemmDesc g) {
                     float4 v = *reinterpret_cast<const float4*>(strip + row * 40 + 4 * (lane & 7));
                     const int m = m0 + ra0 + i * 32 + row;
                     if (m >= g.M || n >= g.N) continue;
+                    if (g.fbias) {  // n is a multiple of 4, the bias of any alignment
+                        v.x += g.fbias[n]; v.y += g.fbias[n + 1];
+                        v.z += g.fbias[n + 2]; v.w += g.fbias[n + 3];
+                    }
                     float* dst = reinterpret_cast<float*>(m < g.Msplit ? g.C : g.C2) +
                                  (size_t)(m < g.Msplit ? m : m - g.Msplit) * g.ldc + n;
                     if (g.accumulate) {
@@ -374,7 +378,7 @@ int resident_blocks() {
 // at least 16 k-tiles (256 k), the partial planes within cap.  Returns the number of
 // non-empty ranges (1: no split).
 int choose_split(const GemmDesc& g, size_t cap) {
-    if (cap == 0 || g.N % 4 || g.ldc % 4 || !al16(g.C) || (g.C2 && !al16(g.C2))) return 1;
+    if (cap == 0 || g.fbias || g.N % 4 || g.ldc % 4 || !al16(g.C) || (g.C2 && !al16(g.C2))) return 1;
     const int tm = wide(g) ? 64 : 128, tn = wide(g) ? 256 : 128;
     const long tiles = (long)((g.M + tm - 1) / tm) * ((g.N + tn - 1) / tn);
     const int KT = k_tiles(g);
@@ -426,6 +430,13 @@ bool gemm_f32_applicable(const GemmDesc& g) {
 size_t gemm_f32_part_bytes(const GemmDesc& g) {
     const int ks = choose_split(g, ~(size_t)0);
     return ks > 1 ? (size_t)ks * g.M * g.N * sizeof(float) : 0;
+}
+
+void gemm_f32_grid(const GemmDesc& g, long& blocks, int& stages) {
+    const int ks = choose_split(g, g.part ? g.part_cap : 0);
+    const int tm = wide(g) ? 64 : 128, tn = wide(g) ? 256 : 128;
+    blocks = (long)((g.M + tm - 1) / tm) * ((g.N + tn - 1) / tn) * ks;
+    stages = (k_tiles(g) + ks - 1) / ks;
 }
 
 int gemm_f32_launch(const GemmDesc& g0, int transA, int transB, hipStream_t s) {

@@ -109,3 +109,52 @@ def test_ffn_ragged_tokens(gn, T, d, H):
     assert err(dX, G @ Wg.double() + U @ Wu.double()) < 2.0 ** -8
     for got, ref in ((dWg, G.t() @ n.double()), (dWu, U.t() @ n.double()), (dbg, G.sum(0)), (dbu, U.sum(0))):
         assert err(got, ref) < 1e-5
+
+
+def guarded32(g, *shape, offset=0):
+    """As guarded, fp32."""
+    n = 1
+    for s in shape:
+        n *= s
+    buf = torch.full((offset + n + 4096,), float("nan"), device="cuda:0")
+    buf[offset:offset + n] = torch.randn(n, device="cuda:0", generator=g)
+    return buf[offset:offset + n].view(*shape)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 129), (33, 31, 161), (64, 256, 784), (64, 10, 256), (163, 88, 1182),
+                                   (6, 163, 1182), (1055, 1023, 300), (30, 50, 2000), (5, 7, 300)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_gemm_fp32_any_size(gn, ta, tb, M, N, K, offset):
+    """fp32 products off the six-product split's sizes, four and eight shares of K, K tails, and
+    unaligned operands; element-wise against a bound of K roundings of the sum of magnitudes."""
+    g = gen(M + N + K)
+    A = guarded32(g, *((K, M) if ta else (M, K)), offset=offset)
+    B = guarded32(g, *((N, K) if tb else (K, N)), offset=offset)
+    a, b = (A.double().t() if ta else A.double()), (B.double().t() if tb else B.double())
+    ref, mag = a @ b, a.abs() @ b.abs()
+    bound = 2.0 ** -24 * (K // 4 + 8)
+    C = gn.gemm(A, B, bool(ta), bool(tb))
+    assert bool(((C.double() - ref).abs() <= bound * mag).all())
+    C = torch.ones(M, N, device="cuda:0")
+    gn.gemm(A, B, bool(ta), bool(tb), C=C, accumulate=True)
+    assert bool(((C.double() - ref - 1).abs() <= bound * (mag + 1)).all())
+
+
+def test_gemm_fp32_two_odd_segments_and_infinities(gn):
+    g = gen(9)
+    A0, B0, A1, B1 = (guarded32(g, 45, 301), guarded32(g, 301, 37), guarded32(g, 45, 9), guarded32(g, 9, 37))
+    ref = A0.double() @ B0.double() + A1.double() @ B1.double()
+    assert err(gn.gemm(A0, B0, A1=A1, B1=B1), ref) < 1e-5
+    A0[3, 5] = float("inf")
+    C = gn.gemm(A0, B0)
+    assert bool(C[3].isinf().all()) and bool(C[[0, 1, 2, 4]].isfinite().all())
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 7, 130), (64, 256, 784), (200, 10, 333), (512, 4100, 256), (40, 12, 64)])
+def test_linear_fwd_fp32_bias(gn, M, N, K):
+    """The column bias in the epilogue of each fp32 kernel (matrix instruction, split, gemm_small)."""
+    g = gen(M)
+    X, W, b = guarded32(g, M, K), guarded32(g, N, K), guarded32(g, N)
+    assert err(gn.linear_fwd(X, W, b), X.double() @ W.double().t() + b.double()) < 1e-5
+    assert err(gn.linear_fwd(X, W), X.double() @ W.double().t()) < 1e-5
