@@ -87,6 +87,11 @@ __global__ __launch_bounds__(256) void row_dot(const T* __restrict__ A, const T*
 
 // ---- MFMA path (bf16, D = 64 or 128) ---------------------------------------------------
 //
+// Per 64-key tile of a key mask (attn_key_bias): nothing masked, some keys biased, or every
+// key masked.  A fully masked tile adds nothing (P = dS = 0), so no kernel visits it: padded
+// batches skip their padding.
+constexpr int kTileBiased = 1, kTileDead = 2;
+
 // Operand tiles are 64 rows x D bf16 kept in LDS in their global orientation (row pitch
 // 2D bytes).  The 16-byte chunk c of tile row r sits at chunk position c ^ tswz<D>(r); for
 // the two fragment reads below (ds_read_b128 of one chunk from 32 consecutive rows, and
@@ -291,7 +296,12 @@ __global__ __launch_bounds__(64 * NW) void attn_dkdv_mfma(
     const float c2 = scale * 1.4426950408889634f;
     // key-padding bias of this lane's key; the wave's 32 keys lie in one 64-key tile
     const int bb = bh / H;
-    const bool kmask = KB && kw0 < S && kt[bb * (Spad / 64) + kw0 / 64];
+    const int kflag = KB && kw0 < S ? kt[bb * (Spad / 64) + kw0 / 64] : 0;
+    const bool kmask = KB && kflag != 0;
+    // keys past S or all masked: this wave has no work; both 64-key tiles so: nor has the block
+    const bool idle = kw0 >= S || (KB && kflag == kTileDead);
+    const bool none = KB && kt[bb * (Spad / 64) + j0 / 64] == kTileDead &&
+                      (j0 + 64 >= S || kt[bb * (Spad / 64) + j0 / 64 + 1] == kTileDead);
     const float kbl = kmask && key < S ? kb[(size_t)bb * Spad + key] : 0.f;
 
     // the block's K and V rows stay in LDS (after the stages) for the whole block
@@ -303,7 +313,7 @@ __global__ __launch_bounds__(64 * NW) void attn_dkdv_mfma(
 
     const uint32_t lds0 = lds_addr(smem);
     const int t0 = causal ? j0 / 64 : 0;
-    const int T = (S + 63) / 64 - t0;
+    const int T = none ? 0 : (S + 63) / 64 - t0;
     TileOffsets<D, NW> oQ, oG;
     oQ.init(tQ.sr, wave);
     oG.init(tG.sr, wave);
@@ -321,14 +331,14 @@ __global__ __launch_bounds__(64 * NW) void attn_dkdv_mfma(
         }
     };
 
-    {
+    if (T > 0) {
         const uint32_t kv = lds0 + STAGES * C::STAGE;
         dma_tile<D, NW>(Kr, tK.sr, j0, S, kv);
         dma_tile<D, NW>(Kr, tK.sr, j0 + 64, S, kv + C::TB);
         dma_tile<D, NW>(V, tV.sr, j0, S, kv + 2 * C::TB);
         dma_tile<D, NW>(V, tV.sr, j0 + 64, S, kv + 3 * C::TB);
+        issue(0);
     }
-    issue(0);
     if (STAGES > 2 && T > 1) issue(1);
     // four waves at D = 64: the wave's K and V fragments (8 per k-step row set, 32 registers)
     // are read from LDS once, after the first tile's barrier, and stay in registers
@@ -352,12 +362,14 @@ __global__ __launch_bounds__(64 * NW) void attn_dkdv_mfma(
         const bf16_t* sG = reinterpret_cast<const bf16_t*>(sb + C::TB);
         const float* sL = reinterpret_cast<const float*>(sb + 2 * C::TB);
         const float* sD = sL + 64;
-        if (kw0 >= S || (causal && kw0 > q0 + 63)) continue;  // every key of the wave masked
-        const bool full = kw0 + 31 < S && q0 + 63 < S && (!causal || kw0 + 31 <= q0);
+        if (idle || (causal && kw0 > q0 + 63)) continue;  // every key of the wave masked
+        // only the causal diagonal needs a mask: rows past S have L = +inf (P = dS = 0), lanes
+        // of keys past S hold a column that is not stored
+        const bool full = !causal || kw0 + 31 <= q0;
 
         // 32-query halves (keeps S, dP, P, dS of one half live).  Masked entries get
-        // S = -inf, hence P = dS = 0 (L and D_i are finite everywhere, padding included);
-        // only tiles on the diagonal or the sequence end evaluate the mask (an empty volatile
+        // S = -inf, hence P = dS = 0;
+        // only tiles on the diagonal evaluate the mask (an empty volatile
         // asm keeps the compiler from speculating the mask into every tile as selects).
 #pragma unroll
         for (int hh = 0; hh < HALVES; ++hh) {
@@ -399,8 +411,7 @@ __global__ __launch_bounds__(64 * NW) void attn_dkdv_mfma(
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int q = q0 + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                    const bool ok = q < S && key < S && (!causal || key <= q);
-                    s[r] = ok ? s[r] : -INFINITY;
+                    s[r] = key <= q ? s[r] : -INFINITY;
                 }
             }
             float pv[16], dv[16];
@@ -475,6 +486,38 @@ struct DqCfg {
     static constexpr int LDS = STAGES * STAGE > EPI ? STAGES * STAGE : EPI;
 };
 
+// The flags of a batch row's key tiles as wave-uniform bit masks, 64 tiles (4096 keys) at a time:
+// one load per window instead of one, exposed, per tile.
+struct TileMask {
+    const int* kt;  // the row's flags, or nullptr: no mask
+    int T;          // tiles the kernel visits
+    int window = -1;
+    unsigned long long biased = 0, dead = 0;
+    __device__ __forceinline__ TileMask(const int* kt_, int T_) : kt(kt_), T(T_) {}
+    __device__ __forceinline__ void look(int it) {
+        if ((it >> 6) == window) return;
+        window = it >> 6;
+        const int t = (it & ~63) + (int)(threadIdx.x & 63);
+        const int f = kt && t < T ? kt[t] : 0;
+        biased = __ballot(f == kTileBiased);
+        dead = __ballot(f == kTileDead);
+    }
+    // the first tile from `it` on that is not fully masked (T: none)
+    __device__ __forceinline__ int live(int it) {
+        while (it < T) {
+            look(it);
+            const unsigned long long m = ~dead >> (it & 63);
+            if (m) return min(it + __builtin_ctzll(m), T);
+            it = (it | 63) + 1;
+        }
+        return T;
+    }
+    __device__ __forceinline__ bool some(int it) {
+        look(it);
+        return (biased >> (it & 63)) & 1;
+    }
+};
+
 // dQ for 128 queries (four waves x 32 queries) of one (batch, head); loops over the key
 // tiles of 64 those queries can see.  Per key tile and wave:
 //   S^T = K Q^T, dP^T = V dO^T    (A = K / V rows from LDS, B = Q / dO fragments in VGPRs)
@@ -518,26 +561,40 @@ __global__ __launch_bounds__(256) void attn_dq_mfma(
     TileOffsets<D> oK, oV;
     oK.init(tK.sr, wave);
     oV.init(tV.sr, wave);
-    auto issue = [&](int it) {
-        const uint32_t sb = lds0 + (it % STAGES) * C::STAGE;
+    static_assert(STAGES == 2, "the loop below alternates between two stages");
+    auto issue = [&](int it, int buf) {
+        const uint32_t sb = lds0 + buf * C::STAGE;
         dma_tile_o<D>(Kr, tK.sr, it * 64, S, sb, wave, oK);
         dma_tile_o<D>(V, tV.sr, it * 64, S, sb + C::TB, wave, oV);
     };
 
-    issue(0);
-    if (STAGES > 2 && T > 1) issue(1);
-    for (int it = 0; it < T; ++it) {
-        if (STAGES > 2 && it + 1 < T) __builtin_amdgcn_s_waitcnt(vmcnt_imm(C::DMA_PER_TILE));
-        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    // tiles in order, fully masked ones left out; the biases of a tile (one key per lane) are loaded
+    // ahead of its DMA, so waiting for them never waits for a younger tile
+    TileMask tm(kt ? kt + (size_t)(bh / H) * (Spad / 64) : nullptr, T);
+    const float* kbr = kb ? kb + (size_t)(bh / H) * Spad : nullptr;
+    float kbn = 0.f;
+    auto fetch = [&](int it, int buf) {
+        if (kbr && tm.some(it)) kbn = kbr[it * 64 + lane];
+        issue(it, buf);
+    };
+    int it = tm.live(0);
+    if (it < T) fetch(it, 0);
+    for (int buf = 0, nx; it < T; it = nx, buf ^= 1) {
+        const bool biased = kbr && tm.some(it);
+        nx = tm.live(it + 1);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        asm volatile("" : "+v"(kbn));  // the biases are in before the next tile's DMA is issued
+        const float kbl = kbn;
         __syncthreads();
-        if (it + STAGES - 1 < T) issue(it + STAGES - 1);
+        if (nx < T) fetch(nx, buf ^ 1);
         const int k0 = it * 64;
-        const unsigned char* sb = smem + (it % STAGES) * C::STAGE;
+        const unsigned char* sb = smem + buf * C::STAGE;
         const bf16_t* sK = reinterpret_cast<const bf16_t*>(sb);
         const bf16_t* sV = reinterpret_cast<const bf16_t*>(sb + C::TB);
         if (qw0 >= S || (causal && k0 > qw0 + 31)) continue;  // every key masked for the wave
-        const bool full = qw0 + 31 < S && k0 + 63 < S && (!causal || k0 + 63 <= qw0);
-        const float* kbt = kb && kt[(bh / H) * (Spad / 64) + it] ? kb + (size_t)(bh / H) * Spad + k0 : nullptr;
+        // (rows past S repeat row S - 1 and are not stored)
+        const bool full = k0 + 63 < S && (!causal || k0 + 63 <= qw0);
+        const int klim = (causal ? min(q, S - 1) : S - 1) - k0 - 4 * h;  // last visible key
 
         // masked entries get S = -inf, hence dS = 0
 #pragma unroll
@@ -562,23 +619,15 @@ __global__ __launch_bounds__(256) void attn_dq_mfma(
             fb[0] = frag_cols<D>(sK, 32 * i, 0);
             if (!full) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int kk = k0 + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                    const bool ok = q < S && kk < S && (!causal || kk <= q);
-                    s[r] = ok ? s[r] : -INFINITY;
-                }
+                for (int r = 0; r < 16; ++r)
+                    s[r] = 32 * i + 8 * (r >> 2) + (r & 3) <= klim ? s[r] : -INFINITY;
             }
             float dv[16];
-            if (kbt) {  // key-padding biases of the 16 keys this lane holds (masked tiles only),
-                        // in score units (scale > 0, checked by the entry points)
+            if (biased) {  // key-padding biases of the 16 keys this lane holds (masked tiles only),
+                           // in score units (scale > 0, checked by the entry points)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const float4 k4 = *reinterpret_cast<const float4*>(kbt + 32 * i + 8 * g + 4 * h);
-                    s[4 * g] += k4.x / c2;
-                    s[4 * g + 1] += k4.y / c2;
-                    s[4 * g + 2] += k4.z / c2;
-                    s[4 * g + 3] += k4.w / c2;
-                }
+                for (int r = 0; r < 16; ++r)
+                    s[r] += __shfl(kbl, 32 * i + 8 * (r >> 2) + 4 * h + (r & 3)) / c2;
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r)
@@ -606,6 +655,12 @@ __global__ __launch_bounds__(256) void attn_dq_mfma(
     store_rows<D>(st, head_base<bf16_t>(tdQ, bh, H), tdQ.sr, qw0, S, scale, rope_mode, cs);
 }
 
+// max over lanes l and l ^ 32
+__device__ __forceinline__ float half_max(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // Forward producing the backward's saved tensors: O and the fp32 row logsumexp (natural
 // log, S scaled), flash-attention2-rope.glsl:165-247 semantics with the causal mask.  One
 // block per (b*h, 128 queries), four waves x 32 queries; K and V tiles of 64 keys arrive by
@@ -618,6 +673,11 @@ __global__ __launch_bounds__(256) void attn_dq_mfma(
 //                    accumulator's row order, B = P^T converted in registers).
 // The epilogue scales by 1/l, transposes each wave's 32 x D block through LDS and writes
 // bf16 rows; LSE = (m + log2 l) ln 2.
+// Bound by each wave's chain per tile (LDS reads, MFMAs, exponentials, DMA and barrier) more than
+// by any one unit.  Measured (us): four fragments in flight instead of one, a lazy rescale and
+// the scale inside the exponent's FMA B4 H16 S2048 D128 causal 109 -> 88 (786 TFLOP/s), B8 H12 S1024 D64
+// 36.6 -> 26.4; S = 1000 (whose last rows sent every tile of their wave down the masked path)
+// 45.5 -> 29.0; with a padding mask 59.4 -> 29.2.
 template <int D, int STAGES>
 __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc tV, TDesc tO,
                                                      float* __restrict__ LSE,
@@ -627,6 +687,7 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
     using C = DqCfg<D, STAGES>;
     extern __shared__ __align__(1024) unsigned char smem[];
     constexpr int NT = D / 32, KS = D / 16;
+    constexpr int RING = 4;  // LDS fragments in flight
     const int nqb = (S + 127) / 128;
     const int bh = blockIdx.x, i0 = (nqb - 1 - (int)blockIdx.y) * 128;  // longest rows first
     const bf16_t* Qr = head_base<const bf16_t>(tQ, bh, H);
@@ -651,92 +712,118 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
     TileOffsets<D> oK, oV;
     oK.init(tK.sr, wave);
     oV.init(tV.sr, wave);
-    auto issue = [&](int it) {
-        const uint32_t sb = lds0 + (it % STAGES) * C::STAGE;
+    static_assert(STAGES == 2, "the loop below alternates between two stages");
+    auto issue = [&](int it, int buf) {
+        const uint32_t sb = lds0 + buf * C::STAGE;
         dma_tile_o<D>(Kr, tK.sr, it * 64, S, sb, wave, oK);
         dma_tile_o<D>(V, tV.sr, it * 64, S, sb + C::TB, wave, oV);
     };
 
-    issue(0);
-    if (STAGES > 2 && T > 1) issue(1);
-    for (int it = 0; it < T; ++it) {
-        if (STAGES > 2 && it + 1 < T) __builtin_amdgcn_s_waitcnt(vmcnt_imm(C::DMA_PER_TILE));
-        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    // tiles in order, fully masked ones left out; the biases of a tile (one key per lane) are loaded
+    // ahead of its DMA, so waiting for them never waits for a younger tile
+    TileMask tm(kt ? kt + (size_t)(bh / H) * (Spad / 64) : nullptr, T);
+    const float* kbr = kb ? kb + (size_t)(bh / H) * Spad : nullptr;
+    float kbn = 0.f;
+    auto fetch = [&](int it, int buf) {
+        if (kbr && tm.some(it)) kbn = kbr[it * 64 + lane];
+        issue(it, buf);
+    };
+    int it = tm.live(0);
+    if (it < T) fetch(it, 0);
+    for (int buf = 0, nx; it < T; it = nx, buf ^= 1) {
+        const bool biased = kbr && tm.some(it);
+        nx = tm.live(it + 1);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        asm volatile("" : "+v"(kbn));  // the biases are in before the next tile's DMA is issued
+        const float kbl = kbn;
         __syncthreads();
-        if (it + STAGES - 1 < T) issue(it + STAGES - 1);
+        if (nx < T) fetch(nx, buf ^ 1);
         const int k0 = it * 64;
-        const unsigned char* sb = smem + (it % STAGES) * C::STAGE;
+        const unsigned char* sb = smem + buf * C::STAGE;
         const bf16_t* sK = reinterpret_cast<const bf16_t*>(sb);
         const bf16_t* sV = reinterpret_cast<const bf16_t*>(sb + C::TB);
         if (qw0 >= S || (causal && k0 > qw0 + 31)) continue;  // every key masked for the wave
-        const bool full = qw0 + 31 < S && k0 + 63 < S && (!causal || k0 + 63 <= qw0);
-        const float* kbt = kb && kt[(bh / H) * (Spad / 64) + it] ? kb + (size_t)(bh / H) * Spad + k0 : nullptr;
+        // (rows past S repeat row S - 1 and are not stored)
+        const bool full = k0 + 63 < S && (!causal || k0 + 63 <= qw0);
+        const int klim = (causal ? min(q, S - 1) : S - 1) - k0 - 4 * h;  // last visible key
 
+        // S^T of the two 32-key halves in turn (independent accumulators), each K fragment
+        // requested RING MFMAs ahead
         f32x16_t sc[2];
+        zero16(sc[0]);
+        zero16(sc[1]);
+        {
+            bf16x8_t fa[RING];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            zero16(sc[i]);
-            bf16x8_t fa[2];
-            fa[0] = frag_rows<D>(sK, 32 * i, 0);
+            for (int j = 0; j < RING; ++j) fa[j] = frag_rows<D>(sK, 32 * (j & 1), j >> 1);
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                if (ks + 1 < KS) fa[(ks + 1) & 1] = frag_rows<D>(sK, 32 * i, ks + 1);
-                sc[i] = mfma32(fa[ks & 1], qf[ks], sc[i]);
+            for (int j = 0; j < 2 * KS; ++j) {
+                sc[j & 1] = mfma32(fa[j % RING], qf[j >> 1], sc[j & 1]);
+                if (j + RING < 2 * KS) fa[j % RING] = frag_rows<D>(sK, 32 * ((j + RING) & 1), (j + RING) >> 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        // scores in base-2 units; masked entries are -inf (P = 0)
+        // the first V fragments travel while the softmax runs
+        bf16x8_t fv[RING];
+#pragma unroll
+        for (int j = 0; j < RING; ++j) fv[j] = frag_cols<D>(sV, 16 * (j / NT), 32 * (j % NT));
+        __builtin_amdgcn_sched_barrier(0);
+
+        // scores to base-2 units, masked entries to -inf (P = 0), on the tiles that need it; the
+        // others keep the raw products and scale inside the exponent's FMA
+        const bool raw = full && !biased && c2 > 0.f;
         float mt = -INFINITY;
+        if (!raw) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float v = sc[i][r] * c2;
-                if (kbt) v += kbt[32 * i + 8 * (r >> 2) + 4 * h + (r & 3)];
-                if (!full) {
-                    const int kk = k0 + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                    const bool ok = q < S && kk < S && (!causal || kk <= q);
-                    v = ok ? v : -INFINITY;
+                for (int r = 0; r < 16; ++r) {
+                    float v = sc[i][r] * c2;
+                    if (biased) v += __shfl(kbl, 32 * i + 8 * (r >> 2) + 4 * h + (r & 3));
+                    if (!full) v = 32 * i + 8 * (r >> 2) + (r & 3) <= klim ? v : -INFINITY;
+                    sc[i][r] = v;
                 }
-                sc[i][r] = v;
-                mt = fmaxf(mt, v);
-            }
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float mn = fmaxf(m, mt);
-        const float ms = mn == -INFINITY ? 0.f : mn;  // a row with no visible key yet stays empty
-        const float alpha = __builtin_amdgcn_exp2f(m - ms);
-        float ps = 0.f;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mt = fmaxf(mt, fmaxf(sc[0][r], sc[1][r]));
+        const float f = raw ? c2 : 1.0f;
+        mt = half_max(mt) * f;
+        // The running maximum moves only when a score exceeds it by more than 2^8: P then stays
+        // below 2^8 (its bf16 and the fp32 sums keep their relative precision), and O and l are
+        // rescaled on the few tiles where some row's maximum has moved instead of on every one.
+        const bool moves = mt > m + 8.0f;
+        if (__any(moves)) {
+            const float mn = moves ? mt : m;
+            const float alpha = moves ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;
+            m = mn;
+            l *= alpha;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) aO[t][r] *= alpha;
+        }
+        const float ms = m == -INFINITY ? 0.f : m;  // a row with no visible key yet stays empty
         bf16x8_t pb[4];
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             float pv[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                pv[e] = __builtin_amdgcn_exp2f(sc[p >> 1][8 * (p & 1) + e] - ms);
-                ps += pv[e];
+                pv[e] = __builtin_amdgcn_exp2f(fmaf(sc[p >> 1][8 * (p & 1) + e], f, -ms));
+                l += pv[e];
             }
             pb[p] = to_bf16x8(pv[0], pv[1], pv[2], pv[3], pv[4], pv[5], pv[6], pv[7]);
         }
-        ps += __shfl_xor(ps, 32);
-        l = l * alpha + ps;
-        m = mn;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) aO[t][r] *= alpha;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            bf16x8_t fv[2];
-            fv[0] = frag_cols<D>(sV, 0, 32 * t);
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                if (p + 1 < 4) fv[(p + 1) & 1] = frag_cols<D>(sV, 16 * (p + 1), 32 * t);
-                aO[t] = mfma32(fv[p & 1], pb[p], aO[t]);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+        for (int j = 0; j < 4 * NT; ++j) {
+            aO[j % NT] = mfma32(fv[j % RING], pb[j / NT], aO[j % NT]);
+            if (j + RING < 4 * NT)
+                fv[j % RING] = frag_cols<D>(sV, 16 * ((j + RING) / NT), 32 * ((j + RING) % NT));
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
+    l += __shfl_xor(l, 32);  // the other 16 keys of every 32
 
     __syncthreads();
     float* st = reinterpret_cast<float*>(smem) + wave * 32 * (D + 4);
@@ -855,7 +942,7 @@ __global__ __launch_bounds__(256) void rope_qk_prep(TDesc tQ, TDesc tK, bf16_t* 
 }
 
 // Pre-pass of the MFMA path, D/8 lanes per row: rotated Q and K (bf16), D_i = rowsum(dO*O)
-// and L log2(e), both into [B*H][Spad] arrays whose padding the kernels never unmask.
+// and L log2(e), both into [B*H][Spad] arrays whose padding gives P = dS = 0.
 template <int D>
 __global__ __launch_bounds__(256) void attn_prep(
     TDesc tQ, TDesc tK, TDesc tG, TDesc tO, const float* __restrict__ LSE, bf16_t* __restrict__ Qr,
@@ -895,16 +982,19 @@ __global__ __launch_bounds__(256) void attn_prep(
     Di[(size_t)bh * Spad + pos] = dot;
     // a row with every visible key masked (LSE = -inf, O = 0) gets P = 0 through L = +inf
     Lsc[(size_t)bh * Spad + pos] = lse == -INFINITY ? INFINITY : lse * 1.4426950408889634f;
-    if (c == 0 && pos == S - 1)  // finite padding: masked entries compute exp2(-inf - 0) * (dP - 0)
-        for (int p = S; p < Spad; ++p) Di[(size_t)bh * Spad + p] = Lsc[(size_t)bh * Spad + p] = 0.f;
+    if (c == 0 && pos == S - 1)  // padding rows the same: P = exp2(s - inf) = 0, dS = 0 (dP - 0)
+        for (int p = S; p < Spad; ++p) {
+            Di[(size_t)bh * Spad + p] = 0.f;
+            Lsc[(size_t)bh * Spad + p] = INFINITY;
+        }
     if (mode == GN_ROPE_NONE) return;
     rotate_qk_chunk<D>(qk4, c, tab, mode, Qr + off, Kr + off);
 }
 
 // Key-padding pre-pass: kb[b][k] = the reference's score bias (mask[b S + k] - 1) 1e9 in
 // base-2 units, -inf where that bias is below -1e4 (exp() of the biased score is then 0 in fp32
-// for any row that keeps a key), 0 past S; kt[b][t] = 1 when 64-key tile t holds a nonzero
-// bias.  One wave per tile.
+// for any row that keeps a key), 0 past S; kt[b][t] = kTileDead when every key of 64-key tile t is
+// masked, else kTileBiased when it holds a nonzero bias, else 0.  One wave per tile.
 __global__ __launch_bounds__(256) void attn_key_bias(const float* __restrict__ mask,
                                                      float* __restrict__ kb, int* __restrict__ kt,
                                                      int B, int S, int Spad) {
@@ -918,8 +1008,8 @@ __global__ __launch_bounds__(256) void attn_key_bias(const float* __restrict__ m
         v = bias < -1e4f ? -INFINITY : bias * 1.4426950408889634f;
     }
     kb[(size_t)b * Spad + k] = v;
-    const unsigned long long any = __ballot(v != 0.f);
-    if (lane == 0) kt[tile] = any != 0ull;
+    const unsigned long long any = __ballot(v != 0.f), live = __ballot(k < S && v != -INFINITY);
+    if (lane == 0) kt[tile] = live == 0ull ? kTileDead : any != 0ull ? kTileBiased : 0;
 }
 
 // ---- generic MFMA path: D a multiple of 32 up to 256, bf16 or fp32 ---------------------
