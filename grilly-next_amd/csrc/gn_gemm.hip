@@ -546,8 +546,10 @@ int gemm_run(const GemmDesc& d, int transA, int transB, int dtype, int c_dtype, 
             return GN_E_INVALID;
         }
         if (small_applicable(d)) return launch_small<float, float>(d, transA, transB, s);
-        if (gemm_f32_applicable(d) && !gemm_f32mm_wins(d)) return gemm_f32_launch(d, transA, transB, s);
-        return gemm_f32mm_launch(d, transA, transB, s);
+        if (gemm_f32_applicable(d))
+            return gemm_f32x6t_wins(d) ? gemm_f32x6t_launch(d, transA, transB, s)
+                                       : gemm_f32_launch(d, transA, transB, s);
+        return gemm_f32seq_launch(d, transA, transB, s);
     }
     set_error("gn_gemm: dtype %d not supported (f32, bf16)", dtype);
     return GN_E_INVALID;

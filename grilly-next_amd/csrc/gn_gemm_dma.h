@@ -95,17 +95,19 @@ int gemm_wave_launch(const GemmDesc& g, int shape, int transA, int transB, int c
 // 16-byte aligned.
 void launch_split_reduce(const GemmDesc& g, hipStream_t s);
 
-// fp32 operands on the fp32 matrix instruction, any size and alignment (gn_gemm_f32mm.hip);
-// _wins: it is faster than the split below for a shape that takes both
-bool gemm_f32mm_wins(const GemmDesc& g);
-int gemm_f32mm_launch(const GemmDesc& g, int transA, int transB, hipStream_t s);
+// fp32 products on small tiles (gn_gemm_f32mm.hip): the fp32 matrix instruction for any size and
+// alignment, and the six-product split below for products that would give it a few blocks
+// (_wins; same bits)
+int gemm_f32seq_launch(const GemmDesc& g, int transA, int transB, hipStream_t s);
+bool gemm_f32x6t_wins(const GemmDesc& g);
+int gemm_f32x6t_launch(const GemmDesc& g, int transA, int transB, hipStream_t s);
 
 // fp32 operands on the bf16 MFMA pipe through a six-product three-piece split (gn_gemm_f32.hip)
 bool gemm_f32_applicable(const GemmDesc& g);
 // workspace bytes the launch would use for split-K partial planes (0: none)
 size_t gemm_f32_part_bytes(const GemmDesc& g);
-// the launch's blocks and 16-k stages per block, for a choice between the fp32 kernels
-void gemm_f32_grid(const GemmDesc& g, long& blocks, int& stages);
+// the launch's blocks, 16-k stages per block and split, for a choice between the fp32 kernels
+void gemm_f32_grid(const GemmDesc& g, long& blocks, int& stages, int& ks);
 int gemm_f32_launch(const GemmDesc& g, int transA, int transB, hipStream_t s);
 
 template <typename CT, int EPI>

@@ -432,8 +432,8 @@ size_t gemm_f32_part_bytes(const GemmDesc& g) {
     return ks > 1 ? (size_t)ks * g.M * g.N * sizeof(float) : 0;
 }
 
-void gemm_f32_grid(const GemmDesc& g, long& blocks, int& stages) {
-    const int ks = choose_split(g, g.part ? g.part_cap : 0);
+void gemm_f32_grid(const GemmDesc& g, long& blocks, int& stages, int& ks) {
+    ks = choose_split(g, g.part ? g.part_cap : 0);
     const int tm = wide(g) ? 64 : 128, tn = wide(g) ? 256 : 128;
     blocks = (long)((g.M + tm - 1) / tm) * ((g.N + tn - 1) / tn) * ks;
     stages = (k_tiles(g) + ks - 1) / ks;

@@ -114,9 +114,8 @@ size_t gn_linear_workspace_bytes(int M, int N, int K, int dtype);
  * dtype GN_BF16: A, B bf16, fp32 accumulation, C is bf16 (c_dtype GN_BF16) or fp32 (GN_F32).
  * dtype GN_F32: all fp32.  Small products (k <= 128 and M*N*k <= 2^24) are plain fp32 FMA
  * chains.  Larger ones with M, N, K multiples of 4 and 16-byte aligned operands run on the
- * bf16 matrix cores, unless K > 256 and their tiles are few; those, other sizes and unaligned
- * operands run on the fp32 matrix instruction (fp32 multiply-adds, inf stays inf).  On the bf16
- * matrix cores each element x is split into three bf16 pieces (|x - x0 - x1 - x2| <=
+ * bf16 matrix cores; other sizes and unaligned operands are fp32 multiply-adds in order of k
+ * (inf stays inf).  On the bf16 matrix cores each element x is split into three bf16 pieces (|x - x0 - x1 - x2| <=
  * 2^-25 |x|) and six piece products are accumulated in fp32, so each product term is within
  * ~2^-24 |a b| (fp32-grade: the sum carries fp32 accumulation error on top).  That path has
  * two documented limits: an inf operand, or one above the bf16 maximum (|x| > 3.3895e38),
