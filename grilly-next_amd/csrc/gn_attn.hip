@@ -39,11 +39,16 @@ namespace gn {
 namespace {
 
 // RoPE angle for pair i at position p: p * base^(-2i/D), reduced in fp64 then sincos fp32.
-__device__ __forceinline__ void rope_cs(int p, int i, int D, float theta, float& c, float& s) {
-    const double inv = exp2(-2.0 * (double)i / (double)D * log2((double)theta));
+__device__ __forceinline__ double rope_inv(int i, int D, float theta) {
+    return exp2(-2.0 * (double)i / (double)D * log2((double)theta));
+}
+__device__ __forceinline__ void rope_cs(int p, double inv, float& c, float& s) {
     double a = (double)p * inv;
     a = a - 6.283185307179586 * rint(a * 0.15915494309189535);
     sincosf((float)a, &s, &c);
+}
+__device__ __forceinline__ void rope_cs(int p, int i, int D, float theta, float& c, float& s) {
+    rope_cs(p, rope_inv(i, D, theta), c, s);
 }
 // pair index i and the two element positions of pair i
 __device__ __forceinline__ void rope_pair(int mode, int i, int D, int& e0, int& e1) {
@@ -1114,8 +1119,31 @@ __device__ __forceinline__ void gen_store(const GenStage<D, NP>& st, unsigned ch
     if (tid < 16) reinterpret_cast<float4*>(sb + C::TILE)[tid] = st.r;
 }
 
-template <int ROLE, int D, int NP, int DC>
-__global__ __launch_bounds__(256) void attn_bwd_gen(GenIn in, const float* __restrict__ L2,
+// Add group 1's accumulators to group 0's through LDS (every wave of the block calls it).
+template <int NT>
+__device__ __forceinline__ void add_groups(unsigned char* smem, int grp, int wave, f32x16_t (&acc)[NT]) {
+    float* p = reinterpret_cast<float*>(smem) + (size_t)wave * NT * 16 * 64 + (threadIdx.x & 63);
+    __syncthreads();
+    if (grp == 1) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) p[(t * 16 + r) * 64] = acc[t][r];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[t][r] += p[(t * 16 + r) * 64];
+    }
+}
+
+// G = 2: two groups of four waves share the block's rows and take every other tile each (own LDS
+// buffers), group 1's sums are added to group 0's at the end: half the chain of tiles per block,
+// for grids that leave CUs idle.
+template <int ROLE, int D, int NP, int DC, int G>
+__global__ __launch_bounds__(256 * G) void attn_bwd_gen(GenIn in, const float* __restrict__ L2,
                                                     const float* __restrict__ Di,
                                                     const float* __restrict__ kb,
                                                     float* __restrict__ outA,
@@ -1125,8 +1153,10 @@ __global__ __launch_bounds__(256) void attn_bwd_gen(GenIn in, const float* __res
     constexpr int KS = D / 16, NT = DC / 32, CR = D / 8;
     extern __shared__ __align__(16) unsigned char smem[];
     const int bh = blockIdx.x, bb = bh / H;
-    const int lane = threadIdx.x & 63, h = lane >> 5, tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, h = lane >> 5, tid = threadIdx.x & 255;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+    const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    unsigned char* const buf = smem + grp * 2 * C::STAGE;
     const int blk = ROLE == 0 ? (int)blockIdx.y : (S + 127) / 128 - 1 - (int)blockIdx.y;
     const int w0 = blk * 128 + 32 * wave, wrow = w0 + (lane & 31);
     const int dcol0 = blockIdx.z * DC;
@@ -1183,13 +1213,14 @@ __global__ __launch_bounds__(256) void attn_bwd_gen(GenIn in, const float* __res
     // T >= 1 (the causal ranges always hold the block's own rows).  The loads and stores run
     // unconditionally (the last iteration re-stages its own tile into the unused buffer), so the
     // staging registers stay registers.
-    gen_load<D, NP>(stg, src, tbeg, S, tid);
-    gen_store<D, NP>(stg, smem, tid);
-    for (int it = 0; it < T; ++it) {
+    gen_load<D, NP>(stg, src, tbeg + 32 * min(grp, T - 1), S, tid);
+    gen_store<D, NP>(stg, buf, tid);
+    for (int j = 0; j < (T + G - 1) / G; ++j) {  // the same count for both groups
+        const int it = grp + G * j;
         __syncthreads();  // tile it is in LDS; the other buffer's readers are done
-        gen_load<D, NP>(stg, src, tbeg + 32 * min(it + 1, T - 1), S, tid);
+        gen_load<D, NP>(stg, src, tbeg + 32 * min(it + G, T - 1), S, tid);
         const int t0 = tbeg + 32 * it;
-        const unsigned char* sb = smem + (it & 1) * C::STAGE;
+        const unsigned char* sb = buf + (j & 1) * C::STAGE;
         const bf16_t* tT[2][NP];
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
@@ -1199,9 +1230,10 @@ __global__ __launch_bounds__(256) void attn_bwd_gen(GenIn in, const float* __res
         const float* srow = reinterpret_cast<const float*>(sb + C::TILE);
         // tile rows t0 .. t0+31 against the wave's rows w0 .. w0+31
         const int q_lo = ROLE == 0 ? t0 : w0, k_lo = ROLE == 0 ? w0 : t0;
-        const bool skip = w0 >= S || (causal && k_lo > q_lo + 31);
+        const bool skip = it >= T || w0 >= S || (causal && k_lo > q_lo + 31);
         if (!skip) {
-            const bool full = t0 + 31 < S && w0 + 31 < S && (!causal || k_lo + 31 <= q_lo);
+            // wave rows past S repeat row S - 1 and are not stored; tile rows past S are masked
+            const bool full = t0 + 31 < S && (!causal || k_lo + 31 <= q_lo);
             f32x16_t s, dp;
             zero16(s);
             zero16(dp);
@@ -1234,7 +1266,7 @@ __global__ __launch_bounds__(256) void attn_bwd_gen(GenIn in, const float* __res
                 float x = s[r] * c2 + br - Lr;
                 if (!full) {
                     const int q = ROLE == 0 ? t0 + tr : wrow, k = ROLE == 0 ? wrow : t0 + tr;
-                    x = (q < S && k < S && (!causal || k <= q)) ? x : -INFINITY;
+                    x = (t0 + tr < S && (!causal || k <= q)) ? x : -INFINITY;
                 }
                 pv[r] = __builtin_amdgcn_exp2f(x);
                 dv[r] = pv[r] * (dp[r] - Dr);
@@ -1265,7 +1297,12 @@ __global__ __launch_bounds__(256) void attn_bwd_gen(GenIn in, const float* __res
                     accB[t] = mma_np<NP>(da[p], c0, accB[t]);
                 }
         }
-        gen_store<D, NP>(stg, smem + ((it + 1) & 1) * C::STAGE, tid);
+        gen_store<D, NP>(stg, buf + ((j + 1) & 1) * C::STAGE, tid);
+    }
+    if constexpr (G == 2) {
+        if constexpr (ROLE == 0) add_groups<NT>(smem, grp, wave, accA);
+        add_groups<NT>(smem, grp, wave, accB);
+        if (grp == 1) return;
     }
 
     // fp32 rows out: column dcol0 + 32t + lane%32, wave rows w0 + 8(r/4) + 4h + r%4
@@ -1290,16 +1327,18 @@ __global__ __launch_bounds__(256) void attn_bwd_gen(GenIn in, const float* __res
 //   transpose reads, B = P^T from the accumulator, both in the accumulator's key order).
 // O = O^T / l leaves in the input dtype, LSE = (m + log2 l) ln 2 (-inf for a row with no visible
 // kept key, whose O is 0).
-template <typename T, int D, int NP>
-__global__ __launch_bounds__(256) void attn_fwd_gen(GenIn in, const float* __restrict__ kb,
+template <typename T, int D, int NP, int G>
+__global__ __launch_bounds__(256 * G) void attn_fwd_gen(GenIn in, const float* __restrict__ kb,
                                                     T* __restrict__ O, float* __restrict__ LSE,
                                                     int H, int S, int Spad, float scale, int causal) {
     using C = GenCfg<D, NP>;
     constexpr int KS = D / 16, NT = D / 32;
     extern __shared__ __align__(16) unsigned char smem[];
     const int bh = blockIdx.x, bb = bh / H;
-    const int lane = threadIdx.x & 63, h = lane >> 5, tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, h = lane >> 5, tid = threadIdx.x & 255;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+    const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    unsigned char* const buf = smem + grp * 2 * C::STAGE;
     const int blk = (S + 127) / 128 - 1 - (int)blockIdx.y;  // longest rows first
     const int w0 = blk * 128 + 32 * wave, q = w0 + (lane & 31);
     const float c2 = scale * 1.4426950408889634f;
@@ -1322,13 +1361,14 @@ __global__ __launch_bounds__(256) void attn_fwd_gen(GenIn in, const float* __res
     GenStage<D, NP> stg;
     const GenSrc src{in.t[1][0], in.t[1][NP - 1], in.t[2][0], in.t[2][NP - 1], kb, nullptr, LSE,
                      (size_t)bb * Spad, hb};
-    gen_load<D, NP>(stg, src, 0, S, tid);
-    gen_store<D, NP>(stg, smem, tid);
-    for (int it = 0; it < Tn; ++it) {
+    gen_load<D, NP>(stg, src, 32 * min(grp, Tn - 1), S, tid);
+    gen_store<D, NP>(stg, buf, tid);
+    for (int j = 0; j < (Tn + G - 1) / G; ++j) {  // the same count for both groups
+        const int it = grp + G * j;
         __syncthreads();
-        gen_load<D, NP>(stg, src, 32 * min(it + 1, Tn - 1), S, tid);
+        gen_load<D, NP>(stg, src, 32 * min(it + G, Tn - 1), S, tid);
         const int k0 = 32 * it;
-        const unsigned char* sb = smem + (it & 1) * C::STAGE;
+        const unsigned char* sb = buf + (j & 1) * C::STAGE;
         const bf16_t* tK[NP];
         const bf16_t* tV[NP];
 #pragma unroll
@@ -1337,8 +1377,9 @@ __global__ __launch_bounds__(256) void attn_fwd_gen(GenIn in, const float* __res
             tV[p] = reinterpret_cast<const bf16_t*>(sb) + (size_t)(NP + p) * 32 * C::P;
         }
         const float* sbias = reinterpret_cast<const float*>(sb + C::TILE);
-        if (!(w0 >= S || (causal && k0 > w0 + 31))) {
-            const bool full = k0 + 31 < S && w0 + 31 < S && (!causal || k0 + 31 <= w0);
+        if (!(it >= Tn || w0 >= S || (causal && k0 > w0 + 31))) {
+            // (rows past S repeat row S - 1 and are not stored)
+            const bool full = k0 + 31 < S && (!causal || k0 + 31 <= w0);
             f32x16_t s;
             zero16(s);
 #pragma unroll
@@ -1360,7 +1401,7 @@ __global__ __launch_bounds__(256) void attn_fwd_gen(GenIn in, const float* __res
                 float v = s[r] * c2 + (kb ? sbias[kr] : 0.f);
                 if (!full) {
                     const int k = k0 + kr;
-                    v = (q < S && k < S && (!causal || k <= q)) ? v : -INFINITY;
+                    v = (k < S && (!causal || k <= q)) ? v : -INFINITY;
                 }
                 x[r] = v;
                 mt = fmaxf(mt, v);
@@ -1400,7 +1441,25 @@ __global__ __launch_bounds__(256) void attn_fwd_gen(GenIn in, const float* __res
                     aO[t] = mma_np<NP>(va, pb[p], aO[t]);
                 }
         }
-        gen_store<D, NP>(stg, smem + ((it + 1) & 1) * C::STAGE, tid);
+        gen_store<D, NP>(stg, buf + ((j + 1) & 1) * C::STAGE, tid);
+    }
+    if constexpr (G == 2) {
+        // both groups to the common maximum, then group 1's sums join group 0's
+        __shared__ float ml[2][2][4][64];
+        ml[grp][0][wave][lane] = m;
+        ml[grp][1][wave][lane] = l;
+        __syncthreads();
+        const float mo = ml[grp ^ 1][0][wave][lane], lo = ml[grp ^ 1][1][wave][lane];
+        const float mn = fmaxf(m, mo), ms = mn == -INFINITY ? 0.f : mn;
+        const float a = __builtin_amdgcn_exp2f(m - ms), ao = __builtin_amdgcn_exp2f(mo - ms);
+        l = grp == 0 ? l * a + lo * ao : l;
+        m = mn;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) aO[t][r] *= a;
+        add_groups<NT>(smem, grp, wave, aO);
+        if (grp == 1) return;
     }
     // O^T accumulators: lane = query, element r of tile t: d = 32t + 8(r/4) + 4h + r%4
     if (q < S) {
@@ -1418,59 +1477,143 @@ __global__ __launch_bounds__(256) void attn_fwd_gen(GenIn in, const float* __res
     }
 }
 
-// Generic path pre-pass: NP bf16 pieces of one [B*H*S, D] tensor (rotated when `mode` is
-// set), one thread per element pair.
+// Four consecutive elements as float, and four floats as consecutive elements (aligned).
+__device__ __forceinline__ float4 ld_quad(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float4 ld_quad(const bf16_t* p) {
+    const uint2 w = *reinterpret_cast<const uint2*>(p);
+    return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u),
+                       __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u));
+}
+__device__ __forceinline__ void st_quad(float* p, const float (&v)[4]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void st_quad(bf16_t* p, const float (&v)[4]) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+}
+
+// Eight elements of a row by unit u (D / 8 units): lo = elements e .. e+3, hi = e2 .. e2+3.  They
+// are consecutive, or in the half-split RoPE mode the two halves of pairs 4u .. 4u+3.
+__device__ __forceinline__ void unit_at(int u, int D, int mode, int& e, int& e2) {
+    e = mode == GN_ROPE_HALF ? 4 * u : 8 * u;
+    e2 = mode == GN_ROPE_HALF ? 4 * u + D / 2 : 8 * u + 4;
+}
+// rotate the unit's four pairs (4u .. 4u+3; inverse: by the opposite angle); inv: the block's table
+// of base^(-2i/D)
+__device__ __forceinline__ void unit_rotate(float (&lo)[4], float (&hi)[4], int u, int pos, int mode,
+                                            bool inverse, const double* inv) {
+    if (mode == GN_ROPE_NONE) return;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        float c, s;
+        rope_cs(pos, inv[4 * u + p], c, s);
+        if (inverse) s = -s;
+        // pair p: (lo[p], hi[p]) in half mode, neighbours 2p, 2p+1 of the eight otherwise
+        float& a = mode == GN_ROPE_HALF ? lo[p] : p < 2 ? lo[2 * (p & 1)] : hi[2 * (p & 1)];
+        float& b = mode == GN_ROPE_HALF ? hi[p] : p < 2 ? lo[2 * (p & 1) + 1] : hi[2 * (p & 1) + 1];
+        const float x0 = a, x1 = b;
+        a = x0 * c - x1 * s;
+        b = x0 * s + x1 * c;
+    }
+}
+__device__ __forceinline__ void rope_inv_table(double* inv, int D, float theta) {
+    for (int i = threadIdx.x; i < D / 2; i += 256) inv[i] = rope_inv(i, D, theta);
+    __syncthreads();
+}
+
+// Generic path pre-pass, one launch: blockIdx.y = tensor to split into NP bf16 pieces (rotated when
+// its mode says so), then (y == n, the backward) the row data D_i = rowsum(dO O) (fp32) and
+// L log2(e), +inf for a row with no visible kept key and for the padding rows (P = dS = 0).
+// Bound by memory at training sizes, by launches at small ones: fp32 B2 H8 S777 D64 with RoPE, seven
+// one-tensor launches and the row pass of the forward and backward took 45 us, two launches here
+// 20.6 us (16-byte accesses, each pair's fp64 angle step once per block).
+struct GenPre {
+    const void* src[4];
+    bf16_t* y[4][2];
+    int mode[4];
+    int n;
+    const void* dO;
+    const void* O;
+    const float* LSE;
+    float* L2;
+    float* Di;
+};
+
 template <typename T, int NP>
-__global__ __launch_bounds__(256) void gen_split(const T* __restrict__ X, bf16_t* __restrict__ y0,
-                                                 bf16_t* __restrict__ y1, int64_t rows, int S,
-                                                 int D, int mode, float theta) {
-    const int half = D / 2;
-    for (int64_t idx = blockIdx.x * (int64_t)256 + threadIdx.x; idx < rows * half;
-         idx += (int64_t)gridDim.x * 256) {
-        const int64_t row = idx / half;
-        const int i = (int)(idx % half);
-        int e0 = 2 * i, e1 = 2 * i + 1;
-        if (mode != GN_ROPE_NONE) rope_pair(mode, i, D, e0, e1);
-        float x0 = io<T>::ld(X, row * D + e0), x1 = io<T>::ld(X, row * D + e1);
-        if (mode != GN_ROPE_NONE) {
-            float c, sn;
-            rope_cs((int)(row % S), i, D, theta, c, sn);
-            const float r0 = x0 * c - x1 * sn, r1 = x0 * sn + x1 * c;
-            x0 = r0;
-            x1 = r1;
+__global__ __launch_bounds__(256) void gen_pre(GenPre g, int64_t BH, int S, int Spad, int D, float theta) {
+    __shared__ double inv[128];  // D <= 256
+    const int j = blockIdx.y;
+    if (j == g.n) {
+        const int lane = threadIdx.x & 63;
+        const T* dO = (const T*)g.dO;
+        const T* O = (const T*)g.O;
+        for (int64_t r = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6); r < BH * Spad; r += (int64_t)gridDim.x * 4) {
+            const int64_t bh = r / Spad;
+            const int pos = (int)(r % Spad);
+            float dot = 0.f;
+            if (pos < S) {
+                const size_t off = ((size_t)bh * S + pos) * D;
+                for (int d = lane; d < D; d += 64) dot += io<T>::ld(dO, off + d) * io<T>::ld(O, off + d);
+            }
+            dot = wave_sum(dot);
+            if (lane == 0) {
+                const float lse = pos < S ? g.LSE[(size_t)bh * S + pos] : -INFINITY;
+                g.Di[r] = dot;
+                g.L2[r] = lse == -INFINITY ? INFINITY : lse * 1.4426950408889634f;
+            }
         }
-        const bf16_t h0 = f2bf(x0), h1 = f2bf(x1);
-        y0[row * D + e0] = h0;
-        y0[row * D + e1] = h1;
+        return;
+    }
+    const int mode = g.mode[j];
+    if (mode != GN_ROPE_NONE) rope_inv_table(inv, D, theta);
+    const T* X = (const T*)g.src[j];
+    const int units = D / 8;
+    const int64_t total = BH * S * units;
+    for (int64_t idx = blockIdx.x * (int64_t)256 + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256) {
+        const int64_t row = idx / units;
+        const int u = (int)(idx % units);
+        int e, e2;
+        unit_at(u, D, mode, e, e2);
+        const float4 a4 = ld_quad(X + row * D + e), b4 = ld_quad(X + row * D + e2);
+        float lo[4] = {a4.x, a4.y, a4.z, a4.w}, hi[4] = {b4.x, b4.y, b4.z, b4.w};
+        unit_rotate(lo, hi, u, (int)(row % S), mode, false, inv);
+        st_quad(g.y[j][0] + row * D + e, lo);
+        st_quad(g.y[j][0] + row * D + e2, hi);
         if (NP == 2) {
-            y1[row * D + e0] = f2bf(x0 - bf2f(h0));
-            y1[row * D + e1] = f2bf(x1 - bf2f(h1));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                lo[i] -= bf2f(f2bf(lo[i]));
+                hi[i] -= bf2f(f2bf(hi[i]));
+            }
+            st_quad(g.y[j][1] + row * D + e, lo);
+            st_quad(g.y[j][1] + row * D + e2, hi);
         }
     }
 }
 
-// Generic path row data: D_i = rowsum(dO O) (fp32) and L log2(e) (+inf for a row with no
-// visible kept key) into [B*H][Spad], padding zero.  One wave per row.
+// fp32 rotated-gradient rows -> output dtype, applying R^T where the tensor's mode says so;
+// blockIdx.y = tensor (D a multiple of 8, aligned: the generic path).
+struct GenPost {
+    const float* acc[2];
+    void* out[2];
+    int mode[2];
+};
 template <typename T>
-__global__ __launch_bounds__(256) void gen_rows(const T* __restrict__ dO, const T* __restrict__ O,
-                                                const float* __restrict__ LSE, float* __restrict__ L2,
-                                                float* __restrict__ Di, int64_t BH, int S, int Spad,
-                                                int D) {
-    const int64_t r = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6);  // padded row index
-    const int lane = threadIdx.x & 63;
-    if (r >= BH * Spad) return;
-    const int64_t bh = r / Spad;
-    const int pos = (int)(r % Spad);
-    float dot = 0.f;
-    if (pos < S) {
-        const size_t off = ((size_t)bh * S + pos) * D;
-        for (int d = lane; d < D; d += 64) dot += io<T>::ld(dO, off + d) * io<T>::ld(O, off + d);
-    }
-    dot = wave_sum(dot);
-    if (lane == 0) {
-        const float lse = pos < S ? LSE[(size_t)bh * S + pos] : 0.f;
-        Di[r] = dot;
-        L2[r] = pos >= S ? 0.f : lse == -INFINITY ? INFINITY : lse * 1.4426950408889634f;
+__global__ __launch_bounds__(256) void gen_post(GenPost g, int64_t rows, int S, int D, float theta) {
+    __shared__ double inv[128];
+    const int j = blockIdx.y, mode = g.mode[j];
+    if (mode != GN_ROPE_NONE) rope_inv_table(inv, D, theta);
+    const int units = D / 8;
+    for (int64_t idx = blockIdx.x * (int64_t)256 + threadIdx.x; idx < rows * units;
+         idx += (int64_t)gridDim.x * 256) {
+        const int64_t row = idx / units;
+        const int u = (int)(idx % units);
+        int e, e2;
+        unit_at(u, D, mode, e, e2);
+        const float4 a4 = ld_quad(g.acc[j] + row * D + e), b4 = ld_quad(g.acc[j] + row * D + e2);
+        float lo[4] = {a4.x, a4.y, a4.z, a4.w}, hi[4] = {b4.x, b4.y, b4.z, b4.w};
+        unit_rotate(lo, hi, u, (int)(row % S), mode, true, inv);
+        st_quad((T*)g.out[j] + row * D + e, lo);
+        st_quad((T*)g.out[j] + row * D + e2, hi);
     }
 }
 
@@ -1795,78 +1938,128 @@ bool allow_gen_lds(F* fn, size_t bytes) {
     return bytes <= 64 * 1024 || allow_lds(fn, bytes);
 }
 
-template <typename T, int D, int NP>
-int launch_gen_bwd(const AttnWs& w, const void* Q, const void* K, const void* V, const void* O,
-                   const void* dO, const float* LSE, const float* mask, void* dQ, void* dK,
-                   void* dV, int B, int H, int S, float scale, int causal, int rope_mode,
-                   float theta, hipStream_t s) {
-    using C = GenCfg<D, NP>;
-    constexpr int DC = D > 128 ? D / 2 : D;
-    static const bool ok0 = allow_gen_lds(attn_bwd_gen<0, D, NP, DC>, C::LDS);
-    static const bool ok1 = allow_gen_lds(attn_bwd_gen<1, D, NP, D>, C::LDS);
-    if (!ok0 || !ok1) {
-        set_error("gn_attn_bwd: cannot reserve %d B of LDS (generic path)", C::LDS);
-        return GN_E_HIP;
-    }
-    const int64_t BH = (int64_t)B * H, rows = BH * S;
-    const int Spad = spad_of(S);
-    const float* kb;
-    const int* kt;
-    key_bias(mask, w, B, S, s, &kb, &kt);
-    GenIn in{};
-    const void* src[4] = {Q, K, V, dO};
-    gen_planes<T, NP>(w, src, 4, in, rows, S, D, rope_mode, theta, s);
-    gen_rows<T><<<(unsigned)((BH * Spad + 3) / 4), 256, 0, s>>>((const T*)dO, (const T*)O, LSE, w.L2,
-                                                                 w.Di, BH, S, Spad, D);
-    const unsigned nb = (unsigned)((S + 127) / 128);
-    hipLaunchKernelGGL((attn_bwd_gen<0, D, NP, DC>), dim3((unsigned)BH, nb, D / DC), dim3(256), C::LDS,
-                       s, in, w.L2, w.Di, kb, w.accA, w.accB, H, S, Spad, scale, causal);
-    const unsigned ge = grid_for(rows * (D / 2), 256, 16384);
-    unrotate_store<T><<<ge, 256, 0, s>>>(w.accB, (T*)dK, rows, S, D, rope_mode, theta);
-    unrotate_store<T><<<ge, 256, 0, s>>>(w.accA, (T*)dV, rows, S, D, GN_ROPE_NONE, theta);
-    hipLaunchKernelGGL((attn_bwd_gen<1, D, NP, D>), dim3((unsigned)BH, nb, 1), dim3(256), C::LDS, s,
-                       in, w.L2, w.Di, kb, nullptr, w.accB, H, S, Spad, scale, causal);
-    unrotate_store<T><<<ge, 256, 0, s>>>(w.accB, (T*)dQ, rows, S, D, rope_mode, theta);
-    GN_LAUNCH_CHECK("gn_attn_bwd (generic mfma)");
-    return GN_OK;
-}
+// Two wave groups per block (G = 2) up to this many blocks: two per CU and below, where each
+// block's chain of tiles is what takes the time.  fp32 D = 64, S = 777, 112 blocks: forward 48 -> 30,
+// dK/dV 63 -> 40, dQ 56 -> 36 us; fp32 B4 H12 S1024 D128, 384 blocks: forward 142 -> 89, backward
+// 470 -> 374 us with the pre-pass (its D = 128 groups spill some registers and still lead).
+constexpr int64_t kGenSplitBlocks = 512;
 
 // operand planes of the generic path: rotated Q, K; V, dO as they are (bf16 inputs without
-// rotation are used in place).  n = 3 for the forward (Q, K, V), 4 for the backward.
+// rotation are used in place).  n = 3 for the forward (Q, K, V), 4 for the backward, which also
+// gets its row data (pre.LSE set).
 template <typename T, int NP>
-void gen_planes(const AttnWs& w, const void* const* src, int n, GenIn& in, int64_t rows, int S,
-                int D, int rope_mode, float theta, hipStream_t s) {
-    const unsigned g = grid_for(rows * (D / 2), 256, 16384);
+int gen_planes(const AttnWs& w, const void* const* src, int n, GenPre& pre, GenIn& in, int64_t BH, int S,
+               int D, int rope_mode, float theta, hipStream_t s) {
+    pre.n = 0;
     for (int i = 0; i < n; ++i) {
         const int mode = i < 2 ? rope_mode : GN_ROPE_NONE;
         if (NP == 1 && mode == GN_ROPE_NONE) {
             in.t[i][0] = in.t[i][1] = (const bf16_t*)src[i];
             continue;
         }
-        gen_split<T, NP><<<g, 256, 0, s>>>((const T*)src[i], w.plane[i][0], w.plane[i][NP - 1], rows,
-                                           S, D, mode, theta);
-        for (int p = 0; p < 2; ++p) in.t[i][p] = w.plane[i][p < NP ? p : 0];
+        for (int p = 0; p < 2; ++p) in.t[i][p] = pre.y[pre.n][p] = w.plane[i][p < NP ? p : 0];
+        pre.src[pre.n] = src[i];
+        pre.mode[pre.n++] = mode;
     }
+    const unsigned jobs = (unsigned)pre.n + (pre.LSE ? 1 : 0);
+    if (jobs == 0) return GN_OK;
+    const unsigned g = grid_for(BH * S * (D / 8), 256, 8192);
+    gen_pre<T, NP><<<dim3(g, jobs), 256, 0, s>>>(pre, BH, S, spad_of(S), D, theta);
+    GN_LAUNCH_CHECK("gn_attn (generic pre-pass)");
+    return GN_OK;
+}
+
+template <int ROLE, int D, int NP, int DC, int G>
+int launch_gen_role(const GenIn& in, const AttnWs& w, const float* kb, float* outA, float* outB, int64_t BH,
+                    int H, int S, float scale, int causal, hipStream_t s) {
+    using C = GenCfg<D, NP>;
+    constexpr size_t lds = (size_t)G * C::LDS;
+    static const bool ok = allow_gen_lds(attn_bwd_gen<ROLE, D, NP, DC, G>, lds);
+    if (!ok) {
+        set_error("gn_attn_bwd: cannot reserve %zu B of LDS (generic path)", lds);
+        return GN_E_HIP;
+    }
+    hipLaunchKernelGGL((attn_bwd_gen<ROLE, D, NP, DC, G>),
+                       dim3((unsigned)BH, (unsigned)((S + 127) / 128), D / DC), dim3(256 * G), lds, s, in, w.L2,
+                       w.Di, kb, outA, outB, H, S, spad_of(S), scale, causal);
+    GN_LAUNCH_CHECK("gn_attn_bwd (generic mfma)");
+    return GN_OK;
+}
+
+template <typename T, int D, int NP>
+int launch_gen_bwd(const AttnWs& w, const void* Q, const void* K, const void* V, const void* O,
+                   const void* dO, const float* LSE, const float* mask, void* dQ, void* dK,
+                   void* dV, int B, int H, int S, float scale, int causal, int rope_mode,
+                   float theta, hipStream_t s) {
+    constexpr int DC = D > 128 ? D / 2 : D, G2 = D <= 128 ? 2 : 1;
+    const int64_t BH = (int64_t)B * H, rows = BH * S;
+    const float* kb;
+    const int* kt;
+    key_bias(mask, w, B, S, s, &kb, &kt);
+    GenIn in{};
+    GenPre pre{};
+    pre.dO = dO; pre.O = O; pre.LSE = LSE; pre.L2 = w.L2; pre.Di = w.Di;
+    const void* src[4] = {Q, K, V, dO};
+    int rc = gen_planes<T, NP>(w, src, 4, pre, in, BH, S, D, rope_mode, theta, s);
+    if (rc) return rc;
+    const bool two = BH * ((S + 127) / 128) <= kGenSplitBlocks;
+    auto dkdv = [&](float* a, float* b) {
+        return two ? launch_gen_role<0, D, NP, DC, G2>(in, w, kb, a, b, BH, H, S, scale, causal, s)
+                   : launch_gen_role<0, D, NP, DC, 1>(in, w, kb, a, b, BH, H, S, scale, causal, s);
+    };
+    auto dq = [&](float* b) {
+        return two ? launch_gen_role<1, D, NP, D, G2>(in, w, kb, nullptr, b, BH, H, S, scale, causal, s)
+                   : launch_gen_role<1, D, NP, D, 1>(in, w, kb, nullptr, b, BH, H, S, scale, causal, s);
+    };
+    auto post = [&](const GenPost& g, unsigned n) {
+        gen_post<T><<<dim3(grid_for(rows * (D / 8), 256, 8192), n), 256, 0, s>>>(g, rows, S, D, theta);
+        GN_LAUNCH_CHECK("gn_attn_bwd (generic output)");
+        return (int)GN_OK;
+    };
+    // fp32 gradients that need no rotation leave the kernels as they are; the others go
+    // through fp32 rows in the workspace
+    if (sizeof(T) == 4) {
+        const bool rope = rope_mode != GN_ROPE_NONE;
+        if ((rc = dkdv((float*)dV, rope ? w.accB : (float*)dK))) return rc;
+        if ((rc = dq(rope ? w.accA : (float*)dQ)) || !rope) return rc;
+        return post(GenPost{{w.accA, w.accB}, {dQ, dK}, {rope_mode, rope_mode}}, 2);
+    }
+    if ((rc = dkdv(w.accA, w.accB))) return rc;
+    if ((rc = post(GenPost{{w.accA, w.accB}, {dV, dK}, {GN_ROPE_NONE, rope_mode}}, 2))) return rc;
+    if ((rc = dq(w.accB))) return rc;
+    return post(GenPost{{w.accB, nullptr}, {dQ, nullptr}, {rope_mode, 0}}, 1);
+}
+
+template <typename T, int D, int NP, int G>
+int launch_gen_fwd_g(const GenIn& in, const float* kb, void* O, float* LSE, int64_t BH, int H, int S, float scale,
+                     int causal, hipStream_t s) {
+    using C = GenCfg<D, NP>;
+    constexpr size_t lds = (size_t)G * C::LDS;
+    static const bool ok = allow_gen_lds(attn_fwd_gen<T, D, NP, G>, lds);
+    if (!ok) {
+        set_error("gn_attn_fwd: cannot reserve %zu B of LDS (generic path)", lds);
+        return GN_E_HIP;
+    }
+    hipLaunchKernelGGL((attn_fwd_gen<T, D, NP, G>), dim3((unsigned)BH, (unsigned)((S + 127) / 128)),
+                       dim3(256 * G), lds, s, in, kb, (T*)O, LSE, H, S, spad_of(S), scale, causal);
+    GN_LAUNCH_CHECK("gn_attn_fwd (generic mfma)");
+    return GN_OK;
 }
 
 template <typename T, int D, int NP>
 int launch_gen_fwd(const AttnWs& w, const void* Q, const void* K, const void* V, const float* kb,
                    void* O, float* LSE, int B, int H, int S, float scale, int causal,
                    int rope_mode, float theta, hipStream_t s) {
-    using C = GenCfg<D, NP>;
-    static const bool ok = allow_gen_lds(attn_fwd_gen<T, D, NP>, C::LDS);
-    if (!ok) {
-        set_error("gn_attn_fwd: cannot reserve %d B of LDS (generic path)", C::LDS);
-        return GN_E_HIP;
-    }
+    constexpr int G2 = D <= 128 ? 2 : 1;
     const int64_t BH = (int64_t)B * H;
     GenIn in{};
+    GenPre pre{};
     const void* src[3] = {Q, K, V};
-    gen_planes<T, NP>(w, src, 3, in, BH * S, S, D, rope_mode, theta, s);
-    hipLaunchKernelGGL((attn_fwd_gen<T, D, NP>), dim3((unsigned)BH, (unsigned)((S + 127) / 128)),
-                       dim3(256), C::LDS, s, in, kb, (T*)O, LSE, H, S, spad_of(S), scale, causal);
-    GN_LAUNCH_CHECK("gn_attn_fwd (generic mfma)");
-    return GN_OK;
+    const int rc = gen_planes<T, NP>(w, src, 3, pre, in, BH, S, D, rope_mode, theta, s);
+    if (rc) return rc;
+    if (BH * ((S + 127) / 128) <= kGenSplitBlocks)
+        return launch_gen_fwd_g<T, D, NP, G2>(in, kb, O, LSE, BH, H, S, scale, causal, s);
+    return launch_gen_fwd_g<T, D, NP, 1>(in, kb, O, LSE, BH, H, S, scale, causal, s);
 }
 
 template <typename T, int NP>
