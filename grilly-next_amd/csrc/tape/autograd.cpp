@@ -43,8 +43,12 @@ inline uint64_t mix(uint64_t x) {
 
 BackwardEngine::BackwardEngine(Device& dev) : dev_(dev), table_(kGradTableSize) { clear_grads(); }
 
+// Only the slots in use: a pass holds tens of entries, and rewriting all 8192 (256 KB) at its begin
+// and end took half of a small step's host time (MLP training step 76 -> 54 us with the
+// front end's own changes).
 void BackwardEngine::clear_grads() {
-    for (auto& e : table_) e = GradEntry{};
+    for (uint32_t i : slots_) table_[i] = GradEntry{};
+    slots_.clear();
     count_ = 0;
 }
 
@@ -66,6 +70,7 @@ BackwardEngine::GradEntry* BackwardEngine::find_or_insert(uint64_t id) {
     size_t i = mix(id) & mask;
     while (table_[i].buffer_id != 0) i = (i + 1) & mask;
     table_[i] = GradEntry{id, 0, 0, 0, false};
+    slots_.push_back((uint32_t)i);
     ++count_;
     return &table_[i];
 }

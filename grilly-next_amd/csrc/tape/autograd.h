@@ -237,6 +237,7 @@ private:
     size_t ws_bytes_ = 0;
     std::vector<uint64_t> backward_bufs_;
     mutable std::vector<GradEntry> table_;
+    std::vector<uint32_t> slots_;  // the table's slots in use
     uint32_t count_ = 0;
     struct FusedSlot {
         uint64_t weight;

@@ -179,22 +179,27 @@ import torch  # noqa: E402  (plumbing: device memory and streams)
 
 
 def _ptr(t):
+    """Device address of a tensor (None -> None); ctypes takes it as the void* it is."""
     if t is None:
         return None
     if not t.is_cuda:
         raise GnError("tensor is not on the GPU")
     if not t.is_contiguous():
         raise GnError("tensor must be contiguous")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _off(t, nbytes):
     """Device address nbytes past the start of t (a column block of a row-major buffer)."""
-    return ctypes.c_void_p(_ptr(t).value + nbytes)
+    return _ptr(t) + nbytes
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current HIP stream's handle.  Asked from torch's C interface: a Stream object per call
+    (torch.cuda.current_stream) took 2.5 us of a small call's 8."""
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dt(t):
@@ -682,9 +687,7 @@ def vsa_cosine_blend_bwd(bits, weights, blended, loss_info, K, grad_scale=10.0):
 
 def _addr(x):
     """Device address of a tensor (its data pointer) or of a raw buffer id (int); None -> 0."""
-    if x is None:
-        return None
-    if isinstance(x, int):
+    if x is None or isinstance(x, int):
         return x
     if not x.is_cuda or not x.is_contiguous():
         raise GnError("optimizer tensors must be contiguous GPU tensors")
@@ -693,20 +696,23 @@ def _addr(x):
 
 def _opt_params(entries):
     arr = (OptParam * max(1, len(entries)))()
+    f32 = torch.float32
     for i, e in enumerate(entries):
         W = e["W"]
-        if W.dtype != torch.float32:
+        if W.dtype != f32:
             raise GnError("optimizer weights (masters) must be float32")
         n = W.numel()
+        get = e.get
+        lp = get("W_bf16")
+        ptrs = [_addr(W)]
         for key in ("grad", "state0", "state1", "recalled"):
-            x = e.get(key)
-            if x is not None and not isinstance(x, int) and (x.numel() != n or x.dtype != torch.float32):
+            x = get(key)
+            if x is not None and not isinstance(x, int) and (x.dtype != f32 or x.numel() != n):
                 raise GnError(f"optimizer tensor {i}: {key} must be float32 with {n} elements")
-        lp = e.get("W_bf16")
+            ptrs.append(_addr(x))
         if lp is not None and (lp.numel() != n or lp.dtype != torch.bfloat16):
             raise GnError(f"optimizer tensor {i}: W_bf16 must be bfloat16 with {n} elements")
-        arr[i] = OptParam(_addr(W), _addr(e["grad"]), _addr(e["state0"]), _addr(e.get("state1")),
-                          _addr(e.get("recalled")), _addr(lp), n)
+        arr[i] = (*ptrs, _addr(lp), n)
     return arr
 
 

@@ -24,24 +24,24 @@ def create_tape_context(device, arena_capacity: int = 64 << 20):
 
 
 def make_tensor_ref(buffer_id: int, shape, dtype: int = DTYPE_F32, requires_grad: bool = False):
-    ref = grilly_core.TensorRef()
-    ref.buffer_id = int(buffer_id)
-    ref.set_shape([int(s) for s in shape])
-    ref.dtype = int(dtype)
-    ref.requires_grad = bool(requires_grad)
-    return ref
+    return grilly_core.TensorRef.of(int(buffer_id), [int(s) for s in shape], int(dtype), bool(requires_grad))
+
+
+_DTYPE_CODES = {}
 
 
 def dtype_code(t) -> int:
-    import torch
-    return {torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16,
-            torch.int32: DTYPE_I32}[t.dtype]
+    if not _DTYPE_CODES:
+        import torch
+        _DTYPE_CODES.update({torch.float32: DTYPE_F32, torch.float16: DTYPE_F16,
+                             torch.bfloat16: DTYPE_BF16, torch.int32: DTYPE_I32})
+    return _DTYPE_CODES[t.dtype]
 
 
 def tref(t, requires_grad: bool = False):
     """TensorRef over a contiguous torch tensor on the GPU (no copy)."""
     assert t.is_cuda and t.is_contiguous()
-    return make_tensor_ref(t.data_ptr(), t.shape, dtype_code(t), requires_grad)
+    return grilly_core.TensorRef.of(t.data_ptr(), t.shape, dtype_code(t), requires_grad)
 
 
 def attach_torch_stream(device):
