@@ -81,8 +81,9 @@ bool gemm_dma_applicable(const GemmDesc& g, int transA, int transB);
 // unbounded (0: none).
 size_t gemm_dma_part_bytes(const GemmDesc& g, int transA, int c_dtype);
 int gemm_dma_launch(const GemmDesc& g, int transA, int transB, int c_dtype, hipStream_t s);
-// Its instantiation units (gn_gemm_dma_{f32a,f32b,bf16,glu}.hip): fp32 C with A k-contiguous /
-// k-outer, bf16 C, and the GLU epilogue (untransposed operands only).
+// Its instantiation units (gn_gemm_dma_{f32a,f32b,glu}.hip): fp32 C with A k-contiguous / k-outer and
+// the GLU epilogue (untransposed operands only); bf16 C (no row sums, one destination) is
+// gn_gemm_stream.hip.
 int gemm_dma_f32_ta0(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_f32_ta1(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s);

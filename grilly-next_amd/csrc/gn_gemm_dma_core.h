@@ -1,7 +1,8 @@
 // gn_gemm_dma_core.h — gfx950 GEMM core: LDS-DMA staging + transpose reads.  Kernel and
 // launch templates (internal linkage); gn_gemm_dma.hip holds the dispatch and the VSA
-// weight-gradient launch, and gn_gemm_dma_{f32a,f32b,bf16,glu}.hip instantiate the GEMM
-// launches per output type / epilogue (/ A orientation), so the builds run in parallel.
+// weight-gradient launch, and gn_gemm_dma_{f32a,f32b,glu}.hip instantiate the GEMM
+// launches per epilogue / A orientation, so the builds run in parallel; bf16 outputs run on
+// gn_gemm_stream.hip, from the same stages and fragments.
 //
 //   C[M x N] (+)= sum_s opA(A_s) opB(B_s)        (up to two K-segments, own leading dims)
 //

@@ -1,0 +1,281 @@
+// gn_gemm_stream.hip — bf16-output products (every operand orientation) on blocks that stay: one
+// per CU, each walking its share of the tiles with the k-tiles of all of them as one stream.
+//
+// A block per tile (gn_gemm_dma_core.h) spends ~11 us on its DMA prologue, pipeline fill and
+// fp32-staged epilogue around the 10 us that 12 k-tiles of a 256 x 128 tile need.  Here the four
+// producer waves run on into the next tile's k-tiles while the four compute waves store the
+// finished one, and the store goes out as bf16 through 4 KB of LDS per wave, so that a tile costs
+// its k-tiles and ~3 us.  What bounds it: at 12 k-tiles the store bursts and the k-tiles about
+// equally, from ~32 k-tiles on the matrix cores and the LDS reads that feed them.
+//   us, a block per tile -> here (A k-contiguous, B row-major [N][K]; in brackets B [K][N]):
+//   8192 x 32000 x 768  689 -> 447 (668 -> 464)    8192 x 3072 x 768   63 -> 42
+//   2001 x 32000 x 768  152 -> 99                  8192 x  768 x 768   19 -> 15 (16 -> 14)
+//   4096 x 5632 x 2048  112 -> 89  (100 -> 87)     8192 x  768 x 6144  78 -> 68 (67 -> 66)
+//   8192 x 8192 x 4096  515 -> 454                 4096 x  768 x 768   10 -> 9.5
+// The main loop, the order of every output's sum and its roundings are those of the core: the
+// results are the same bits.
+#include <algorithm>
+
+#include "gn_gemm_dma_core.h"
+
+namespace gn {
+namespace {
+
+template <bool TA, bool TB, int BM, int BN, int STAGES>
+__global__ __launch_bounds__(512, 1) void gemm_stream(GemmDesc g) {
+    constexpr int NW = 4;
+    constexpr int A_ELEMS = BM * BK, B_ELEMS = BN * BK, STAGE_B = (A_ELEMS + B_ELEMS) * 2;
+    constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 32, FN = WN / 32, NM = FM * FN;
+    constexpr int RA = TA ? 2 : 1, RB = TB ? 1 : 2, NR = FM * RA + FN * RB;
+    constexpr int NDA = BM / (8 * NW), NDB = BN / (8 * NW), ND = NDA + NDB;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const uint32_t lds0 = lds_addr(smem_raw);
+
+    const int tilesM = (g.M + BM - 1) / BM, tilesN = (g.N + BN - 1) / BN;
+    const int nblk = tilesM * tilesN;
+    const int ntile = (nblk - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;  // this block's
+    // its i-th tile: block b runs on XCD b % 8, each XCD walks one contiguous range of the tiles,
+    // GROUP tile rows at a time (gridDim.x is a
+    // multiple of 8, or the tiles are one round)
+    auto tile_at = [&](int i, int& m0, int& n0) __attribute__((always_inline)) {
+        const int x = (int)blockIdx.x + i * (int)gridDim.x;
+        const int xcd = x & 7, per = nblk >> 3, extra = nblk & 7;
+        const int pid = xcd * per + min(xcd, extra) + (x >> 3);
+        constexpr int GROUP = BM == 256 ? 4 : 8;
+        const int first_m = (pid / (GROUP * tilesN)) * GROUP;
+        const int gsize = min(tilesM - first_m, GROUP);
+        const int in_group = pid % (GROUP * tilesN);
+        m0 = (first_m + in_group % gsize) * BM;
+        n0 = (in_group / gsize) * BN;
+    };
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = (wave >> 1) & 1, wn = wave & 1, dw = wave & 3;
+    const int kt0 = (g.Ks[0] + BK - 1) / BK;
+    const int KT = kt0 + (g.nseg > 1 ? (g.Ks[1] + BK - 1) / BK : 0);
+    const int J = ntile * KT;  // k-tiles of the stream
+
+    if (wave >= 4) {
+        // producers: the compute waves' barriers, the DMA of k-tile j + STAGES after each
+        uint32_t voa[NDA], vob[NDB];
+        int pi = 0, pt = 0, m0, n0, oseg = -1;  // next k-tile to move
+        tile_at(0, m0, n0);
+        auto next = [&](int slot) __attribute__((always_inline)) {
+            const bool s1 = pt >= kt0;
+            const int k0 = (s1 ? pt - kt0 : pt) * BK, klim = s1 ? g.Ks[1] : g.Ks[0];
+            const bf16_t* A = g.A[s1];
+            const bf16_t* B = g.B[s1];
+            const int lda = g.lda[s1], ldb = g.ldb[s1];
+            const uint32_t base = lds0 + (uint32_t)(slot * STAGE_B);
+            if (k0 + BK > klim) {
+                stage_tail<BM, !TA, NW>(A, lda, m0, g.M, k0, klim, dw, base);
+                stage_tail<BN, TB, NW>(B, ldb, n0, g.N, k0, klim, dw, base + A_ELEMS * 2);
+            } else {
+                if (oseg != (int)s1) {
+                    oseg = s1;
+                    stage_offsets<BM, !TA, NW>(lda, m0, g.M, dw, voa);
+                    stage_offsets<BN, TB, NW>(ldb, n0, g.N, dw, vob);
+                }
+                const bf16_t* sa = stage_base<!TA>(A, lda, m0, k0);
+                const bf16_t* sb = stage_base<TB>(B, ldb, n0, k0);
+#pragma unroll
+                for (int q = 0; q < NDA; ++q) dma16s(sa, voa[q], base + 1024u * (uint32_t)(dw * NDA + q));
+#pragma unroll
+                for (int q = 0; q < NDB; ++q)
+                    dma16s(sb, vob[q], base + A_ELEMS * 2 + 1024u * (uint32_t)(dw * NDB + q));
+            }
+            if (++pt == KT) {
+                if (pi + 1 < ntile) {
+                    pt = 0;
+                    tile_at(++pi, m0, n0);
+                    oseg = -1;  // row and column clamps are the tile's
+                } else {
+                    pt = KT - 1;  // past the end: the last k-tile again
+                }
+            }
+        };
+        static_for<STAGES>([&](auto S_) { next(decltype(S_)::value); });
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 1) * ND));
+        __syncthreads();
+        int slot = 0;
+        for (int j = 0; j < J; ++j) {
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 2) * ND));  // k-tile j + 1 has landed
+            __syncthreads();
+            next(slot);
+            slot = slot == STAGES - 1 ? 0 : slot + 1;
+        }
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        return;
+    }
+
+    f32x16_t acc[FM][FN];
+    bf16x8_t fa[4][FM], fb[4][FN];
+    auto read_one = [&](auto SET_, auto R_, const bf16_t* sa, int ks) {
+        constexpr int set = decltype(SET_)::value, r = decltype(R_)::value;
+        if constexpr (r < FM * RA) {
+            if constexpr (r % RA == 0) fa[set][r / RA] = frag<BM, !TA>(sa, wm * WM + (r / RA) * 32, ks);
+        } else {
+            constexpr int rb = r - FM * RA;
+            if constexpr (rb % RB == 0) fb[set][rb / RB] = frag<BN, TB>(sa + A_ELEMS, wn * WN + (rb / RB) * 32, ks);
+        }
+    };
+    auto kstep = [&](auto CUR_, auto RSET_, auto FRONT_, const bf16_t* rsrc, int rks) {
+        constexpr int cur = decltype(CUR_)::value;
+        constexpr bool front = decltype(FRONT_)::value;
+        static_for<NM>([&](auto Q_) {
+            constexpr int q = decltype(Q_)::value;
+            acc[q / FN][q % FN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[cur][q % FN], fa[cur][q / FN],
+                                                                          acc[q / FN][q % FN], 0, 0, 0);
+            constexpr int r0 = reads_before<NM, NR, front>(q), r1 = reads_before<NM, NR, front>(q + 1);
+            static_for<NR>([&](auto R_) {
+                constexpr int r = decltype(R_)::value;
+                if constexpr (r >= r0 && r < r1) read_one(RSET_, R_, rsrc, rks);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    using BF = std::false_type;
+    using BT = std::true_type;
+    auto stage_ptr = [&](int slot) { return reinterpret_cast<const bf16_t*>(smem_raw + slot * STAGE_B); };
+
+    // Store one finished tile.  The products are transposed (op(B)'s fragment first): element r of
+    // a 32 x 32 block is row lane % 32, column 8 (r / 4) + 4 (lane / 32) + r % 4, so four
+    // consecutive elements are four columns of one row.  32 rows at a time go through the wave's
+    // own LDS as bf16 (16-byte chunk c of row m at c ^ (m % 8)) and leave as 128-byte row segments.
+    bf16_t* const C = reinterpret_cast<bf16_t*>(g.C);
+    unsigned char* const st = smem_raw + STAGES * STAGE_B + wave * 4096;
+    auto store = [&](auto MIX_, int m0, int n0) {
+        constexpr bool MIX = decltype(MIX_)::value;  // + cbias, + C
+        int ln = lane;  // opaque: its addresses are formed here, not kept across the k loop
+        asm volatile("" : "+v"(ln));
+        const int mr = ln & 31, nh = 4 * (ln >> 5);
+        const int nw = n0 + wn * WN;
+        const bool nok = nw + (ln & 7) * 8 < g.N;
+        const uint32_t voff = (uint32_t)((ln >> 3) * g.ldc + (ln & 7) * 8) * 2u;
+        static_for<FM>([&](auto I_) {
+            constexpr int i = decltype(I_)::value;
+            const int mw = m0 + wm * WM + i * 32;
+            bf16_t* const Cw = C + (size_t)mw * g.ldc + nw;
+            wave_lds_sync();
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    float v[4];
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) v[d] = acc[i][j][4 * q + d];
+                    if constexpr (MIX) {
+                        const int nc = j * 32 + q * 8 + nh;
+                        if (g.cbias && nw + nc < g.N) {
+                            const uint2 b = *reinterpret_cast<const uint2*>(g.cbias + nw + nc);
+                            v[0] += __uint_as_float(b.x << 16);
+                            v[1] += __uint_as_float(b.x & 0xffff0000u);
+                            v[2] += __uint_as_float(b.y << 16);
+                            v[3] += __uint_as_float(b.y & 0xffff0000u);
+                        }
+                        if (g.accumulate && nw + nc < g.N && mw + mr < g.M) {
+                            const uint2 o = *reinterpret_cast<const uint2*>(Cw + (size_t)mr * g.ldc + nc);
+                            v[0] += __uint_as_float(o.x << 16);
+                            v[1] += __uint_as_float(o.x & 0xffff0000u);
+                            v[2] += __uint_as_float(o.y << 16);
+                            v[3] += __uint_as_float(o.y & 0xffff0000u);
+                        }
+                    }
+                    *reinterpret_cast<uint2*>(st + mr * 128 + (((j * 4 + q) ^ (mr & 7)) * 16) + nh * 2) =
+                        make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            wave_lds_sync();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = q * 8 + (ln >> 3);
+                const uint4 v = *reinterpret_cast<const uint4*>(st + r * 128 + (((ln & 7) ^ (ln >> 3)) * 16));
+                char* dst = reinterpret_cast<char*>(Cw + (size_t)(q * 8) * g.ldc) + voff;
+                if (mw + r < g.M && nok) *reinterpret_cast<uint4*>(dst) = v;
+            }
+        });
+    };
+
+    __syncthreads();  // k-tile 0
+    static_for<NR>([&](auto R_) { read_one(I0{}, R_, stage_ptr(0), 0); });
+    static_for<NR>([&](auto R_) { read_one(I1{}, R_, stage_ptr(0), 1); });
+    int slot = 0;
+    for (int i = 0; i < ntile; ++i) {
+#pragma unroll
+        for (int a = 0; a < FM; ++a)
+#pragma unroll
+            for (int b = 0; b < FN; ++b) zero16(acc[a][b]);
+        for (int t = 0; t < KT; ++t) {
+            const bf16_t* cur = stage_ptr(slot);
+            slot = slot == STAGES - 1 ? 0 : slot + 1;
+            const bf16_t* nxt = stage_ptr(slot);
+            kstep(I0{}, I2{}, BF{}, cur, 2);
+            kstep(I1{}, I3{}, BT{}, cur, 3);
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(63) & 0xF0FFu);  // lgkmcnt(0): cur has no reader left
+            __syncthreads();
+            kstep(I2{}, I0{}, BF{}, nxt, 0);  // the next tile's k-tile 0 after the last
+            kstep(I3{}, I1{}, BF{}, nxt, 1);
+        }
+        int m0, n0;
+        tile_at(i, m0, n0);
+        if (g.cbias || g.accumulate)
+            store(BT{}, m0, n0);
+        else
+            store(BF{}, m0, n0);
+    }
+}
+
+template <bool TA, bool TB, int BM>
+int launch(const GemmDesc& g, int cus, hipStream_t s) {
+    constexpr int BN = 128, STAGES = 3;
+    constexpr size_t smem = (size_t)STAGES * (BM + BN) * BK * sizeof(bf16_t) + 4 * 4096;  // 160 KB at 256 rows
+    static_assert(smem <= 160 * 1024, "LDS per CU");
+    static const bool ok = allow_lds(gemm_stream<TA, TB, BM, BN, STAGES>, smem);
+    if (!ok) {
+        set_error("gemm: cannot reserve %zu B of LDS", smem);
+        return GN_E_HIP;
+    }
+    const long tiles = (long)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
+    hipLaunchKernelGGL((gemm_stream<TA, TB, BM, BN, STAGES>), dim3((unsigned)std::min<long>(tiles, cus)),
+                       dim3(512), smem, s, g);
+    GN_LAUNCH_CHECK("gemm (streamed tiles)");
+    return GN_OK;
+}
+
+// compute units of the current device, rounded down to a multiple of 8 (one block each)
+int stream_blocks() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        cus = 256;
+    return std::max(8, cus / 8 * 8);
+}
+
+template <int BM>
+int launch_tile(const GemmDesc& g, int transA, int transB, int cus, hipStream_t s) {
+    if (!transA && !transB) return launch<false, false, BM>(g, cus, s);
+    if (!transA && transB) return launch<false, true, BM>(g, cus, s);
+    if (transA && !transB) return launch<true, false, BM>(g, cus, s);
+    return launch<true, true, BM>(g, cus, s);
+}
+
+}  // namespace
+
+// 256 x 128 or 128 x 128 tiles, whichever needs less time for its rounds: a round of the small
+// ones takes 0.6 of a round of the large (a k-tile 0.42 against 0.67 us, fixed 4.5 against 7 us).
+// Measured, 256 -> 128 rows: 4096 x 768 x 3072 (one round either way) 33 -> 24 us, 2048^3 24.5 ->
+// 20.2; 8192 x 768 x 3072 (one round against two) 39 -> 48, 2816 x 2304 x 768 14 -> 16.
+int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s) {
+    const int cus = stream_blocks();
+    const long tn = (g.N + 127) / 128;
+    const long r256 = ((g.M + 255) / 256 * tn + cus - 1) / cus, r128 = ((g.M + 127) / 128 * tn + cus - 1) / cus;
+    return 0.62 * (double)r128 < (double)r256 ? launch_tile<128>(g, transA, transB, cus, s)
+                                              : launch_tile<256>(g, transA, transB, cus, s);
+}
+
+}  // namespace gn
