@@ -791,10 +791,10 @@ class Step:
          "4096x5632x2048 (the SwiGLU backward in the GEMM's epilogue)",
          "gemm_core 256x256 (fp32 C) + gemm_core (epi 1) on the side stream", "mfma",
          2.0 * DM * HID * T + 2.0 * T * HID * DM),
-        ("dN = [dG|dU] [Wg;Wu], 4096x2048x11264", "gemm_core 256x128 with producer waves (bf16 C)",
+        ("dN = [dG|dU] [Wg;Wu], 4096x2048x11264", "gemm_stream 256x128 (bf16 C; one block per CU)",
          "mfma", 2.0 * T * DM * 2 * HID),
         ("[dWg;dWu] = [dG|dU]^T N, 11264x2048x4096",
-         "gemm_core 256x128 with producer waves (fp32 C; 704 blocks)", "mfma", 2.0 * 2 * HID * DM * T),
+         "gemm_stream 256x128 (fp32 C; 704 tiles, one block per CU)", "mfma", 2.0 * 2 * HID * DM * T),
         ("RMSNorm backward 4096x2048 (rows + parameter partials)", "norm_bwd_rows + colsum_partials",
          "hbm", 3.0 * T * DM * 2 + 4.0 * T),
     ]

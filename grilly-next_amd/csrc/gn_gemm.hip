@@ -566,8 +566,9 @@ int colsum_dispatch(const void* in, float* out, int M, int N, int dtype, unsigne
 // overwrites) unless accumulating.
 int weight_grad(const void* dY, int ldy, const void* X, int ldx, int M, int N, int Kin, void* dW,
                 void* dW2, int Msplit, float* db, float* db2, int dtype, unsigned flags,
-                hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0) {
+                hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0, bool beside = false) {
     GemmDesc d{};
+    d.beside = beside;
     // split-K partial planes need 16-byte aligned storage; a misaligned workspace is unused
     if (ws && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0) {
         d.part = (float*)ws;
@@ -861,7 +862,7 @@ extern "C" int gn_linear_bwd_ws(const void* dY, const void* X, const void* W, vo
     SideBySide sb(s, dX ? side_by_side(dtype, 2.0 * mac, 2.0 * mac, M, K, N, K) : Fork::kNever);
     // dW[N x K] = dY^T . X  (A = dY stored [M x N] = [Ks x Mout], transposed), db fused
     int rc = weight_grad(dY, N, X, K, M, N, K, dW, dW, N, (float*)db, nullptr, dtype, flags, s, ws,
-                         ws_bytes);
+                         ws_bytes, sb.side() != s);
     if (rc == GN_OK && dX)  // dX[M x K] = dY[M x N] . W[N x K]
         rc = gemm_dispatch(dY, W, N, nullptr, nullptr, 0, dX, M, K, 0, 0, dtype, dtype, flags,
                            sb.side(), dtype == GN_F32 ? ws : nullptr, ws_bytes);
@@ -928,10 +929,10 @@ static int glu_proj_impl(const void* gu, const void* X, const void* Wg, const vo
                                      scr, (size_t)H * K);
             if (rc == GN_OK)
                 rc = weight_grad(g0, 2 * H, X, K, M, 2 * H, K, dWg, dWu, H, nullptr, nullptr, dtype,
-                                 flags, s, ws, ws_bytes);
+                                 flags, s, ws, ws_bytes, sb.side() != s);
         } else {
             rc = weight_grad(g0, 2 * H, X, K, M, 2 * H, K, dWg, dWu, H, (float*)dbg, (float*)dbu,
-                             dtype, flags, s, ws, ws_bytes);
+                             dtype, flags, s, ws, ws_bytes, sb.side() != s);
         }
     }
     if (rc == GN_OK && dX) {
@@ -995,7 +996,7 @@ static int ffn_down_glu_impl(int kind, const void* dY, const void* A, const void
     // frozen down projection (dWd NULL): the local gradients only
     if (dWd)
         rc = weight_grad(dY, N, A, H, M, N, H, dWd, dWd, N, (float*)dbd, nullptr, dtype, flags, s, ws,
-                         ws_bytes);
+                         ws_bytes, sb.side() != s);
     if (rc == GN_OK) {
         GemmDesc d{};
         d.nseg = 1;

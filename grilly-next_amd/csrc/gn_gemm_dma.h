@@ -46,6 +46,8 @@ struct GemmDesc {
     const bf16_t* cbias;
     // the same for an fp32 product (fp32 operands and C, overwritten); nullptr: none
     const float* fbias;
+    // another product shares the GPU with this one (a call's side-by-side pair)
+    bool beside;
     // split-K through a workspace (plain fp32 epilogue, ksplit >= 3): split y stores its
     // partial tile at part + y*M*N (row-major, pitch N) and, with a bias, its row sums at
     // part + ksplit*M*N + y*M; split_reduce then adds the splits in index order into C and
@@ -88,6 +90,9 @@ int gemm_dma_f32_ta0(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_f32_ta1(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s);
 int gemm_dma_glu(const GemmDesc& g, int transA, int transB, hipStream_t s);
+// fp32 C of an unbiased weight gradient (transA, plain epilogue) on streamed tiles, where it wins
+bool gemm_stream_f32_wins(const GemmDesc& g, int transA, int transB);
+int gemm_stream_f32(const GemmDesc& g, hipStream_t s);
 // Small tiles with K split over a block's waves (gn_gemm_wave.hip), for products that the core's
 // tiles would spread over too few compute units: the tile shape to run g on, or -1 (the core).
 int gemm_wave_shape(const GemmDesc& g, int transA, int transB, int c_dtype);

@@ -71,6 +71,7 @@ int gemm_dma_launch(const GemmDesc& g, int transA, int transB, int c_dtype, hipS
     const int wave = gemm_wave_shape(g, transA, transB, c_dtype);
     if (wave >= 0) return gemm_wave_launch(g, wave, transA, transB, c_dtype, s);
     if (g.epi == 1) return gemm_dma_glu(g, transA, transB, s);
+    if (c_dtype == GN_F32 && gemm_stream_f32_wins(g, transA, transB)) return gemm_stream_f32(g, s);
     if (c_dtype == GN_F32) return transA ? gemm_dma_f32_ta1(g, transB, s) : gemm_dma_f32_ta0(g, transB, s);
     return gemm_dma_bf16(g, transA, transB, s);
 }

@@ -1,10 +1,11 @@
-// gn_gemm_stream.hip — bf16-output products (every operand orientation) on blocks that stay: one
-// per CU, each walking its share of the tiles with the k-tiles of all of them as one stream.
+// gn_gemm_stream.hip — bf16-output products (every operand orientation) and the fp32 weight gradients
+// of several rounds on blocks that stay: one per CU, each walking its share of the tiles with the
+// k-tiles of all of them as one stream.
 //
 // A block per tile (gn_gemm_dma_core.h) spends ~11 us on its DMA prologue, pipeline fill and
 // fp32-staged epilogue around the 10 us that 12 k-tiles of a 256 x 128 tile need.  Here the four
 // producer waves run on into the next tile's k-tiles while the four compute waves store the
-// finished one, and the store goes out as bf16 through 4 KB of LDS per wave, so that a tile costs
+// finished one, and the store goes out through 4 KB of LDS per wave, so that a tile costs
 // its k-tiles and ~3 us.  What bounds it: at 12 k-tiles the store bursts and the k-tiles about
 // equally, from ~32 k-tiles on the matrix cores and the LDS reads that feed them.
 //   us, a block per tile -> here (A k-contiguous, B row-major [N][K]; in brackets B [K][N]):
@@ -21,7 +22,7 @@
 namespace gn {
 namespace {
 
-template <bool TA, bool TB, int BM, int BN, int STAGES>
+template <bool TA, bool TB, typename CT, int BM, int BN, int STAGES>
 __global__ __launch_bounds__(512, 1) void gemm_stream(GemmDesc g) {
     constexpr int NW = 4;
     constexpr int A_ELEMS = BM * BK, B_ELEMS = BN * BK, STAGE_B = (A_ELEMS + B_ELEMS) * 2;
@@ -35,8 +36,7 @@ __global__ __launch_bounds__(512, 1) void gemm_stream(GemmDesc g) {
     const int nblk = tilesM * tilesN;
     const int ntile = (nblk - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;  // this block's
     // its i-th tile: block b runs on XCD b % 8, each XCD walks one contiguous range of the tiles,
-    // GROUP tile rows at a time (gridDim.x is a
-    // multiple of 8, or the tiles are one round)
+    // GROUP tile rows at a time (gridDim.x is a multiple of 8, or the tiles are one round)
     auto tile_at = [&](int i, int& m0, int& n0) __attribute__((always_inline)) {
         const int x = (int)blockIdx.x + i * (int)gridDim.x;
         const int xcd = x & 7, per = nblk >> 3, extra = nblk & 7;
@@ -201,6 +201,44 @@ __global__ __launch_bounds__(512, 1) void gemm_stream(GemmDesc g) {
         });
     };
 
+    // fp32 C: one 32 x 32 block at a time, its rows 128 bytes; rows from Msplit on go to C2.
+    auto store32 = [&](auto ACC_, int m0, int n0) {
+        constexpr bool ACC = decltype(ACC_)::value;  // + C
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int mr = ln & 31, c8 = ln & 7, r8 = ln >> 3;
+        static_for<FM>([&](auto I_) {
+            constexpr int i = decltype(I_)::value;
+            const int mw = m0 + wm * WM + i * 32;
+            static_for<FN>([&](auto J_) {
+                constexpr int j = decltype(J_)::value;
+                const int n = n0 + wn * WN + j * 32 + c8 * 4;
+                wave_lds_sync();
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<float4*>(st + mr * 128 + (((2 * q + (ln >> 5)) ^ (mr & 7)) * 16)) =
+                        make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
+                                    acc[i][j][4 * q + 3]);
+                wave_lds_sync();
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int r = q * 8 + r8, m = mw + r;
+                    float4 v = *reinterpret_cast<const float4*>(st + r * 128 + ((c8 ^ r8) * 16));
+                    if (m < g.M && n < g.N) {
+                        float4* dst = reinterpret_cast<float4*>(
+                            reinterpret_cast<float*>(m < g.Msplit ? g.C : g.C2) +
+                            (size_t)(m < g.Msplit ? m : m - g.Msplit) * g.ldc + n);
+                        if constexpr (ACC) {
+                            const float4 o = *dst;
+                            v = make_float4(v.x + o.x, v.y + o.y, v.z + o.z, v.w + o.w);
+                        }
+                        *dst = v;
+                    }
+                }
+            });
+        });
+    };
+
     __syncthreads();  // k-tile 0
     static_for<NR>([&](auto R_) { read_one(I0{}, R_, stage_ptr(0), 0); });
     static_for<NR>([&](auto R_) { read_one(I1{}, R_, stage_ptr(0), 1); });
@@ -223,25 +261,28 @@ __global__ __launch_bounds__(512, 1) void gemm_stream(GemmDesc g) {
         }
         int m0, n0;
         tile_at(i, m0, n0);
-        if (g.cbias || g.accumulate)
-            store(BT{}, m0, n0);
-        else
-            store(BF{}, m0, n0);
+        if constexpr (sizeof(CT) == 4) {
+            if (g.accumulate) store32(BT{}, m0, n0);
+            else store32(BF{}, m0, n0);
+        } else {
+            if (g.cbias || g.accumulate) store(BT{}, m0, n0);
+            else store(BF{}, m0, n0);
+        }
     }
 }
 
-template <bool TA, bool TB, int BM>
+template <bool TA, bool TB, int BM, typename CT = bf16_t>
 int launch(const GemmDesc& g, int cus, hipStream_t s) {
     constexpr int BN = 128, STAGES = 3;
     constexpr size_t smem = (size_t)STAGES * (BM + BN) * BK * sizeof(bf16_t) + 4 * 4096;  // 160 KB at 256 rows
     static_assert(smem <= 160 * 1024, "LDS per CU");
-    static const bool ok = allow_lds(gemm_stream<TA, TB, BM, BN, STAGES>, smem);
+    static const bool ok = allow_lds(gemm_stream<TA, TB, CT, BM, BN, STAGES>, smem);
     if (!ok) {
         set_error("gemm: cannot reserve %zu B of LDS", smem);
         return GN_E_HIP;
     }
     const long tiles = (long)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
-    hipLaunchKernelGGL((gemm_stream<TA, TB, BM, BN, STAGES>), dim3((unsigned)std::min<long>(tiles, cus)),
+    hipLaunchKernelGGL((gemm_stream<TA, TB, CT, BM, BN, STAGES>), dim3((unsigned)std::min<long>(tiles, cus)),
                        dim3(512), smem, s, g);
     GN_LAUNCH_CHECK("gemm (streamed tiles)");
     return GN_OK;
@@ -276,6 +317,21 @@ int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s) {
     const long r256 = ((g.M + 255) / 256 * tn + cus - 1) / cus, r128 = ((g.M + 127) / 128 * tn + cus - 1) / cus;
     return 0.62 * (double)r128 < (double)r256 ? launch_tile<128>(g, transA, transB, cus, s)
                                               : launch_tile<256>(g, transA, transB, cus, s);
+}
+
+// More than two rounds of 256 x 128 tiles, alone on the GPU.  Measured (us, a block per tile -> here, M x N x K
+// of dW): 11264 x 2048 x 4096 178 -> 159, x 2048 112 -> 91, x 300 55 -> 32; 32000 x 768 x 2001 120 -> 95;
+// 8192 x 8192 x 4096 555 -> 472; the least gain just above the line (10240 x 1792 x 4096, 560 tiles,
+// 153 -> 149).  Beside another product (an LM head's dX, 48 tiles over K = 32000) blocks that stay keep it
+// waiting: the pair's pass 522 -> 532, so there the core's blocks go on sharing the GPU.
+bool gemm_stream_f32_wins(const GemmDesc& g, int transA, int transB) {
+    if (!transA || transB || g.bias || g.cbias || g.beside) return false;
+    const long tiles = (long)((g.M + 255) / 256) * ((g.N + 127) / 128);
+    return tiles > 2L * stream_blocks();
+}
+
+int gemm_stream_f32(const GemmDesc& g, hipStream_t s) {
+    return launch<true, false, 256, float>(g, stream_blocks(), s);
 }
 
 }  // namespace gn

@@ -57,3 +57,37 @@ def test_streamed_two_segments(gn, K0, K1):
     A0, B0, A1, B1 = guarded(g, M, K0), guarded(g, K0, N), guarded(g, M, K1), guarded(g, K1, N)
     ref = A0.double() @ B0.double() + A1.double() @ B1.double()
     assert err(gn.gemm(A0, B0, A1=A1, B1=B1, out_dtype=BF), ref) < 2.0 ** -8
+
+
+# fp32 weight gradients of more than two rounds of 256-row tiles (cut by both edges), K tails
+@pytest.mark.parametrize("M,N,K", [(8200, 2056, 8), (8200, 2056, 200), (16392, 1032, 1003), (130, 131080, 64)])
+def test_streamed_weight_gradient(gn, M, N, K):
+    """|sum| error: fp32 accumulation of exact bf16 products, K 2^-24 of the largest term sum."""
+    g = gen(M + K)
+    A, B = guarded(g, K, M - M % 8), guarded(g, K, N)
+    m = A.shape[1]
+    ref = A.double().t() @ B.double()
+    buf = torch.full((m + 8, N), 7.0, device="cuda:0")
+    gn.gemm(A, B, True, False, C=buf[:m])
+    tol = max(K, 64) * 2.0 ** -23
+    assert err(buf[:m], ref) < tol
+    assert bool((buf[m:] == 7).all())
+    C = torch.full((m, N), 2.0, device="cuda:0")
+    gn.gemm(A, B, True, False, C=C, accumulate=True)
+    assert err(C, ref + 2) < tol
+
+
+def test_streamed_weight_gradient_rows_split(gn):
+    """[dWg; dWu] as one product: the second matrix begins inside a tile row."""
+    g = gen(5)
+    T, H, K = 203, 5000, 2056
+    dO, gate, up, n = guarded(g, T, H), guarded(g, T, H), guarded(g, T, H), guarded(g, T, K)
+    Wg, Wu = guarded(g, H, K), guarded(g, H, K)
+    _, dWg, dWu, _, _ = gn.glu_linear_bwd("reglu_up", dO, gate, up, n, Wg, Wu)
+    on = (up > 0).double()
+    dg = (dO.double() * up.double() * on).to(BF).double()
+    du = (dO.double() * gate.double() * on).to(BF).double()
+    # the kernel forms each local gradient in fp32 and rounds once, as here: 2^-8 covers an
+    # element that a double rounding moves
+    assert err(dWg, dg.t() @ n.double()) < 2.0 ** -8
+    assert err(dWu, du.t() @ n.double()) < 2.0 ** -8
