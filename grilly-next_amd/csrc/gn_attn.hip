@@ -679,8 +679,8 @@ __device__ __forceinline__ float half_max(float v) {
 // The epilogue scales by 1/l, transposes each wave's 32 x D block through LDS and writes
 // bf16 rows; LSE = (m + log2 l) ln 2.
 // Bound by each wave's chain per tile (LDS reads, MFMAs, exponentials, DMA and barrier) more than
-// by any one unit.  Measured (us): four fragments in flight instead of one, a lazy rescale and
-// the scale inside the exponent's FMA B4 H16 S2048 D128 causal 109 -> 88 (786 TFLOP/s), B8 H12 S1024 D64
+// by any one unit.  Measured (us): four fragments in flight instead of one, O rescaled only
+// where a maximum moved and the scale inside the exponent's FMA B4 H16 S2048 D128 causal 109 -> 88 (786 TFLOP/s), B8 H12 S1024 D64
 // 36.6 -> 26.4; S = 1000 (whose last rows sent every tile of their wave down the masked path)
 // 45.5 -> 29.0; with a padding mask 59.4 -> 29.2.
 template <int D, int STAGES>
@@ -777,7 +777,6 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
         // scores to base-2 units, masked entries to -inf (P = 0), on the tiles that need it; the
         // others keep the raw products and scale inside the exponent's FMA
         const bool raw = full && !biased && c2 > 0.f;
-        float mt = -INFINITY;
         if (!raw) {
 #pragma unroll
             for (int i = 0; i < 2; ++i)
@@ -789,25 +788,24 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
                     sc[i][r] = v;
                 }
         }
+        float mt = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 16; ++r) mt = fmaxf(mt, fmaxf(sc[0][r], sc[1][r]));
         const float f = raw ? c2 : 1.0f;
-        mt = half_max(mt) * f;
-        // The running maximum moves only when a score exceeds it by more than 2^8: P then stays
-        // below 2^8 (its bf16 and the fp32 sums keep their relative precision), and O and l are
-        // rescaled on the few tiles where some row's maximum has moved instead of on every one.
-        const bool moves = mt > m + 8.0f;
-        if (__any(moves)) {
-            const float mn = moves ? mt : m;
-            const float alpha = moves ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;
-            m = mn;
-            l *= alpha;
+        // The maximum is the row's own after every tile, so that a row's leading weight is exactly 1
+        // in bf16: one that lags behind (O and l then rescaled on few tiles) rounds every weight of
+        // the row, and the errors of the leading ones do not average out.
+        const float mn = fmaxf(m, half_max(mt) * f);
+        const float ms = mn == -INFINITY ? 0.f : mn;  // a row with no visible key yet stays empty
+        const float alpha = __builtin_amdgcn_exp2f(m - ms);
+        if (__any(mn > m)) {
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) aO[t][r] *= alpha;
         }
-        const float ms = m == -INFINITY ? 0.f : m;  // a row with no visible key yet stays empty
+        m = mn;
+        float ps[4];  // the tile's sum in four chains, then onto the row's
         bf16x8_t pb[4];
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -815,10 +813,11 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 pv[e] = __builtin_amdgcn_exp2f(fmaf(sc[p >> 1][8 * (p & 1) + e], f, -ms));
-                l += pv[e];
+                ps[p] = e == 0 ? pv[0] : ps[p] + pv[e];
             }
             pb[p] = to_bf16x8(pv[0], pv[1], pv[2], pv[3], pv[4], pv[5], pv[6], pv[7]);
         }
+        l = l * alpha + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < 4 * NT; ++j) {

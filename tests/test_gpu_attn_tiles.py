@@ -1,6 +1,6 @@
 """GPU tests of the bf16 attention kernels' tile selection: key masks that empty whole 64-key tiles
 (which the kernels skip), windows of more than 64 tiles, ragged sequence ends, and maxima that
-grow along a row (the forward rescales only when a maximum moves by more than 2^8).
+grow along a row (the forward rescales O on the tiles where some row's maximum moves).
 
 Tolerance 2e-2 of the largest entry: bf16 probabilities and operands (2^-8), as the other bf16
 attention tests."""
