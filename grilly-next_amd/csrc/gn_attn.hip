@@ -482,13 +482,12 @@ __global__ __launch_bounds__(64 * NW) void attn_dkdv_mfma(
     finish(aK, head_base<bf16_t>(tdK, bh, H), tdK.sr, scale, rope_mode);
 }
 
-template <int D, int STAGES>
+template <int D>
 struct DqCfg {
     static constexpr int TB = tile_bytes(D);
-    static constexpr int STAGE = 2 * TB;  // K tile, V tile
-    static constexpr int DMA_PER_TILE = 2 * (D / 32);
+    static constexpr int STAGE = 2 * TB;  // K tile, V tile; two stages
     static constexpr int EPI = 4 * 32 * (D + 4) * 4;
-    static constexpr int LDS = STAGES * STAGE > EPI ? STAGES * STAGE : EPI;
+    static constexpr int LDS = 2 * STAGE > EPI ? 2 * STAGE : EPI;
 };
 
 // The flags of a batch row's key tiles as wave-uniform bit masks, 64 tiles (4096 keys) at a time:
@@ -529,13 +528,13 @@ struct TileMask {
 //   dS^T = P^T (dP^T - D_i)       (each lane owns one query: its L and D_i are scalars)
 //   dQ += dS K                    (A = dS from the accumulators, B = K columns by
 //                                  transpose reads)
-template <int D, int STAGES>
+template <int D, bool KB>
 __global__ __launch_bounds__(256) void attn_dq_mfma(
     TDesc tQ, TDesc tK, TDesc tV, TDesc tG, const float* __restrict__ Lsc,
     const float* __restrict__ Di, const float2* __restrict__ cs, const float* __restrict__ kb,
     const int* __restrict__ kt, TDesc tdQ, int H, int S, int Spad, float scale, int causal,
     int rope_mode) {
-    using C = DqCfg<D, STAGES>;
+    using C = DqCfg<D>;
     extern __shared__ __align__(1024) unsigned char smem[];
     constexpr int NT = D / 32, KS = D / 16;
     const int nqb = (S + 127) / 128;
@@ -566,29 +565,29 @@ __global__ __launch_bounds__(256) void attn_dq_mfma(
     TileOffsets<D> oK, oV;
     oK.init(tK.sr, wave);
     oV.init(tV.sr, wave);
-    static_assert(STAGES == 2, "the loop below alternates between two stages");
     auto issue = [&](int it, int buf) {
         const uint32_t sb = lds0 + buf * C::STAGE;
         dma_tile_o<D>(Kr, tK.sr, it * 64, S, sb, wave, oK);
         dma_tile_o<D>(V, tV.sr, it * 64, S, sb + C::TB, wave, oV);
     };
 
-    // tiles in order, fully masked ones left out; the biases of a tile (one key per lane) are loaded
-    // ahead of its DMA, so waiting for them never waits for a younger tile
-    TileMask tm(kt ? kt + (size_t)(bh / H) * (Spad / 64) : nullptr, T);
-    const float* kbr = kb ? kb + (size_t)(bh / H) * Spad : nullptr;
+    // Tiles in order.  With a key mask (KB) the fully masked ones are left out, and the biases of a
+    // tile (one key per lane) are loaded ahead of its DMA, so waiting for them never waits for a
+    // younger tile.
+    TileMask tm(KB ? kt + (size_t)(bh / H) * (Spad / 64) : nullptr, T);
+    const float* kbr = KB ? kb + (size_t)(bh / H) * Spad : nullptr;
     float kbn = 0.f;
     auto fetch = [&](int it, int buf) {
-        if (kbr && tm.some(it)) kbn = kbr[it * 64 + lane];
+        if (KB && tm.some(it)) kbn = kbr[it * 64 + lane];
         issue(it, buf);
     };
-    int it = tm.live(0);
+    int it = KB ? tm.live(0) : 0;
     if (it < T) fetch(it, 0);
     for (int buf = 0, nx; it < T; it = nx, buf ^= 1) {
-        const bool biased = kbr && tm.some(it);
-        nx = tm.live(it + 1);
+        const bool biased = KB && tm.some(it);
+        nx = KB ? tm.live(it + 1) : it + 1;
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        asm volatile("" : "+v"(kbn));  // the biases are in before the next tile's DMA is issued
+        if (KB) asm volatile("" : "+v"(kbn));  // the biases are in before the next tile's DMA is issued
         const float kbl = kbn;
         __syncthreads();
         if (nx < T) fetch(nx, buf ^ 1);
@@ -679,17 +678,17 @@ __device__ __forceinline__ float half_max(float v) {
 // The epilogue scales by 1/l, transposes each wave's 32 x D block through LDS and writes
 // bf16 rows; LSE = (m + log2 l) ln 2.
 // Bound by each wave's chain per tile (LDS reads, MFMAs, exponentials, DMA and barrier) more than
-// by any one unit.  Measured (us): four fragments in flight instead of one, O rescaled only
-// where a maximum moved and the scale inside the exponent's FMA B4 H16 S2048 D128 causal 109 -> 88 (786 TFLOP/s), B8 H12 S1024 D64
-// 36.6 -> 26.4; S = 1000 (whose last rows sent every tile of their wave down the masked path)
-// 45.5 -> 29.0; with a padding mask 59.4 -> 29.2.
-template <int D, int STAGES>
+// by any one unit.  Measured (us, replayed): four fragments in flight instead of one, O rescaled only
+// where a maximum moved, the scale inside the exponent's FMA and no mask code without a mask (KB)
+// B4 H16 S2048 D128 causal 106 -> 87, B8 H12 S1024 D64 37 -> 27; S = 1000 (whose last rows sent every
+// tile of their wave down the masked path) 42 -> 27; with a padding mask 56 -> 30.
+template <int D, bool KB>
 __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc tV, TDesc tO,
                                                      float* __restrict__ LSE,
                                                      const float* __restrict__ kb,
                                                      const int* __restrict__ kt, int H, int S,
                                                      int Spad, float scale, int causal) {
-    using C = DqCfg<D, STAGES>;
+    using C = DqCfg<D>;
     extern __shared__ __align__(1024) unsigned char smem[];
     constexpr int NT = D / 32, KS = D / 16;
     constexpr int RING = 4;  // LDS fragments in flight
@@ -717,29 +716,29 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
     TileOffsets<D> oK, oV;
     oK.init(tK.sr, wave);
     oV.init(tV.sr, wave);
-    static_assert(STAGES == 2, "the loop below alternates between two stages");
     auto issue = [&](int it, int buf) {
         const uint32_t sb = lds0 + buf * C::STAGE;
         dma_tile_o<D>(Kr, tK.sr, it * 64, S, sb, wave, oK);
         dma_tile_o<D>(V, tV.sr, it * 64, S, sb + C::TB, wave, oV);
     };
 
-    // tiles in order, fully masked ones left out; the biases of a tile (one key per lane) are loaded
-    // ahead of its DMA, so waiting for them never waits for a younger tile
-    TileMask tm(kt ? kt + (size_t)(bh / H) * (Spad / 64) : nullptr, T);
-    const float* kbr = kb ? kb + (size_t)(bh / H) * Spad : nullptr;
+    // Tiles in order.  With a key mask (KB) the fully masked ones are left out, and the biases of a
+    // tile (one key per lane) are loaded ahead of its DMA, so waiting for them never waits for a
+    // younger tile.
+    TileMask tm(KB ? kt + (size_t)(bh / H) * (Spad / 64) : nullptr, T);
+    const float* kbr = KB ? kb + (size_t)(bh / H) * Spad : nullptr;
     float kbn = 0.f;
     auto fetch = [&](int it, int buf) {
-        if (kbr && tm.some(it)) kbn = kbr[it * 64 + lane];
+        if (KB && tm.some(it)) kbn = kbr[it * 64 + lane];
         issue(it, buf);
     };
-    int it = tm.live(0);
+    int it = KB ? tm.live(0) : 0;
     if (it < T) fetch(it, 0);
     for (int buf = 0, nx; it < T; it = nx, buf ^= 1) {
-        const bool biased = kbr && tm.some(it);
-        nx = tm.live(it + 1);
+        const bool biased = KB && tm.some(it);
+        nx = KB ? tm.live(it + 1) : it + 1;
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        asm volatile("" : "+v"(kbn));  // the biases are in before the next tile's DMA is issued
+        if (KB) asm volatile("" : "+v"(kbn));  // the biases are in before the next tile's DMA is issued
         const float kbl = kbn;
         __syncthreads();
         if (nx < T) fetch(nx, buf ^ 1);
@@ -1789,7 +1788,7 @@ struct AttnWs {
     float2* cs;   // MFMA path: RoPE cos/sin table [S][D/2]
     float* acc;   // SIMT path: fp32 [B*H*S*D]
     float* kb;    // key-padding bias (base 2) [B][Spad] (sized for B*H rows)
-    int* kt;      // per 64-key tile: any key biased [B][Spad/64]
+    int* kt;      // per 64-key tile: 0, kTileBiased or kTileDead [B][Spad/64]
 };
 
 
@@ -1859,7 +1858,7 @@ bool allow_lds(F* fn, size_t bytes) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
 }
 
-constexpr int kStagesDkdv = 2, kStagesDq = 2;
+constexpr int kStagesDkdv = 2;
 // dK/dV waves per block: eight (two per SIMD, one block per CU) at D = 128, where the block's
 // 128 K and V rows and two stages fill the LDS; four at D = 64 (65 KB of LDS, 207 registers),
 // so two blocks share a CU and each wave keeps its K and V fragments in registers
@@ -1883,10 +1882,10 @@ int launch_mfma_bwd(const AttnWs& w, const AttnIO& io, const float* LSE, const f
                     hipStream_t s) {
     constexpr int NWK = dkdv_waves<D>();
     using C1 = DkdvCfg<D, kStagesDkdv, NWK>;
-    using C2 = DqCfg<D, kStagesDq>;
+    using C2 = DqCfg<D>;
     static const bool ok1 = allow_lds(attn_dkdv_mfma<D, kStagesDkdv, NWK, false>, C1::LDS) &&
                             allow_lds(attn_dkdv_mfma<D, kStagesDkdv, NWK, true>, C1::LDS);
-    static const bool ok2 = allow_lds(attn_dq_mfma<D, kStagesDq>, C2::LDS);
+    static const bool ok2 = allow_lds(attn_dq_mfma<D, false>, C2::LDS) && allow_lds(attn_dq_mfma<D, true>, C2::LDS);
     if (!ok1 || !ok2) {
         set_error("gn_attn_bwd: cannot reserve LDS (%d / %d B)", C1::LDS, C2::LDS);
         return GN_E_HIP;
@@ -1921,11 +1920,26 @@ int launch_mfma_bwd(const AttnWs& w, const AttnIO& io, const float* LSE, const f
     hipLaunchKernelGGL(dkdv, dim3(BH, nb), dim3(64 * NWK), C1::LDS, s, tQ, tK, io.V,
                        io.dO, w.Lsc, w.Di, w.cs, kb, kt, io.dK, io.dV, H, S, Spad, scale, causal,
                        rope_mode);
-    hipLaunchKernelGGL((attn_dq_mfma<D, kStagesDq>), dim3(BH, nb), dim3(256), C2::LDS, sb.side(),
+    const auto dq = kb ? attn_dq_mfma<D, true> : attn_dq_mfma<D, false>;
+    hipLaunchKernelGGL(dq, dim3(BH, nb), dim3(256), C2::LDS, sb.side(),
                        tQ, tK, io.V, io.dO, w.Lsc, w.Di, w.cs, kb, kt, io.dQ, H, S, Spad, scale,
                        causal, rope_mode);
     GN_LAUNCH_CHECK("gn_attn_bwd (mfma)");
     return sb.join();
+}
+
+template <int D>
+int launch_mfma_fwd(const TDesc& tQ, const TDesc& tK, const TDesc& tV, const TDesc& tO, float* LSE,
+                    const float* kb, const int* kt, int BH, int H, int S, float scale, int causal,
+                    hipStream_t s) {
+    using C = DqCfg<D>;
+    static const bool ok = allow_lds(attn_fwd_mfma<D, false>, C::LDS) && allow_lds(attn_fwd_mfma<D, true>, C::LDS);
+    GN_REQUIRE(ok, "gn_attn_fwd: cannot reserve %d B of LDS", C::LDS);
+    const auto fwd = kb ? attn_fwd_mfma<D, true> : attn_fwd_mfma<D, false>;
+    hipLaunchKernelGGL(fwd, dim3(BH, (S + 127) / 128), dim3(256), C::LDS, s, tQ, tK, tV, tO, LSE, kb, kt, H, S,
+                       spad_of(S), scale, causal);
+    GN_LAUNCH_CHECK("gn_attn_fwd (mfma)");
+    return GN_OK;
 }
 
 // head dims of the generic MFMA path (multiples of 32 whose dK/dV column groups of <= 128
@@ -2360,22 +2374,8 @@ extern "C" int gn_attn_fwd_mask(const void* Q, const void* K, const void* V, con
         const int BH = B * H;
         const TDesc tQ = bhsd(Qp, H, S, D), tK = bhsd(Kp, H, S, D), tV = bhsd(V, H, S, D),
                     tO = bhsd(O, H, S, D);
-        const dim3 grid(BH, (S + 127) / 128);
-        if (D == 64) {
-            using C = DqCfg<64, kStagesDq>;
-            static const bool ok = allow_lds(attn_fwd_mfma<64, kStagesDq>, C::LDS);
-            GN_REQUIRE(ok, "gn_attn_fwd: cannot reserve %d B of LDS", C::LDS);
-            hipLaunchKernelGGL((attn_fwd_mfma<64, kStagesDq>), grid, dim3(256), C::LDS, s, tQ, tK, tV, tO,
-                               LSE, kb, kt, H, S, Spad, scale, causal);
-        } else {
-            using C = DqCfg<128, kStagesDq>;
-            static const bool ok = allow_lds(attn_fwd_mfma<128, kStagesDq>, C::LDS);
-            GN_REQUIRE(ok, "gn_attn_fwd: cannot reserve %d B of LDS", C::LDS);
-            hipLaunchKernelGGL((attn_fwd_mfma<128, kStagesDq>), grid, dim3(256), C::LDS, s, tQ, tK, tV, tO,
-                               LSE, kb, kt, H, S, Spad, scale, causal);
-        }
-        GN_LAUNCH_CHECK("gn_attn_fwd (mfma)");
-        return GN_OK;
+        return D == 64 ? launch_mfma_fwd<64>(tQ, tK, tV, tO, LSE, kb, kt, BH, H, S, scale, causal, s)
+                       : launch_mfma_fwd<128>(tQ, tK, tV, tO, LSE, kb, kt, BH, H, S, scale, causal, s);
     }
     const unsigned gr = (unsigned)((rows + 3) / 4);
     if (dtype == GN_BF16)
