@@ -1951,11 +1951,22 @@ bool allow_gen_lds(F* fn, size_t bytes) {
     return bytes <= 64 * 1024 || allow_lds(fn, bytes);
 }
 
-// Two wave groups per block (G = 2) up to this many blocks: two per CU and below, where each
-// block's chain of tiles is what takes the time.  fp32 D = 64, S = 777, 112 blocks: forward 48 -> 30,
-// dK/dV 63 -> 40, dQ 56 -> 36 us; fp32 B4 H12 S1024 D128, 384 blocks: forward 142 -> 89, backward
-// 470 -> 374 us with the pre-pass (its D = 128 groups spill some registers and still lead).
-constexpr int64_t kGenSplitBlocks = 512;
+// Two wave groups per block (G = 2)?  They halve a block's chain of tiles, which is what takes the
+// time where a CU has one block, or two of different length (causal).  Two blocks of full rows per CU
+// hide each other's latency as they are, and one or two tiles leave nothing to share.  Measured (us,
+// one group -> two): fp32 D = 64, 112 blocks, S = 777: forward 48 -> 37, backward 121 -> 88; 384 causal
+// blocks, S = 1024: 73 -> 55, 173 -> 127; the same not causal: 77 -> 90, 206 -> 230; 512 blocks, S = 130:
+// 24 -> 30, 56 -> 65.  bf16 D = 96: 384 causal blocks 52 -> 34, 134 -> 107; not causal 68 -> 77, 160 -> 183;
+// 512 blocks, S = 130: 10.9 -> 15.7.  D = 32 is short enough per tile to gain further out (384 blocks not
+// causal, forward 59 -> 50; bf16 backward 112 -> 105, fp32 149 -> 162), as do the fp32 backwards at D = 96
+// (396 -> 371).  Those of D = 128 in two groups do not fit their registers (dK/dV 80 of them spill, dQ
+// 28) and are level from S = 512 (356 against 356 at 384 causal blocks, 690 -> 638 not causal), slower below.
+bool gen_two_groups(int D, bool f32, bool bwd, int64_t blocks, int S, bool causal) {
+    if (S <= (bwd ? 64 : 32)) return false;
+    if (bwd && D == 128) return S >= 512 && blocks <= (causal ? 384 : 512);
+    const bool twice = D == 32 && !bwd ? true : S >= 256 && (causal || (D == 32 ? !f32 : bwd && f32 && D == 96));
+    return blocks <= (twice ? 512 : 256);
+}
 
 // operand planes of the generic path: rotated Q, K; V, dO as they are (bf16 inputs without
 // rotation are used in place).  n = 3 for the forward (Q, K, V), 4 for the backward, which also
@@ -1976,7 +1987,9 @@ int gen_planes(const AttnWs& w, const void* const* src, int n, GenPre& pre, GenI
     }
     const unsigned jobs = (unsigned)pre.n + (pre.LSE ? 1 : 0);
     if (jobs == 0) return GN_OK;
-    const unsigned g = grid_for(BH * S * (D / 8), 256, 8192);
+    // enough blocks for the tensors' units (eight elements a thread) and the row data (a wave a row)
+    const int64_t threads = std::max<int64_t>(pre.n ? BH * S * (D / 8) : 0, pre.LSE ? BH * spad_of(S) * 64 : 0);
+    const unsigned g = grid_for(threads, 256, 8192);
     gen_pre<T, NP><<<dim3(g, jobs), 256, 0, s>>>(pre, BH, S, spad_of(S), D, theta);
     GN_LAUNCH_CHECK("gn_attn (generic pre-pass)");
     return GN_OK;
@@ -2015,7 +2028,7 @@ int launch_gen_bwd(const AttnWs& w, const void* Q, const void* K, const void* V,
     const void* src[4] = {Q, K, V, dO};
     int rc = gen_planes<T, NP>(w, src, 4, pre, in, BH, S, D, rope_mode, theta, s);
     if (rc) return rc;
-    const bool two = BH * ((S + 127) / 128) <= kGenSplitBlocks;
+    const bool two = gen_two_groups(D, sizeof(T) == 4, true, BH * ((S + 127) / 128), S, causal);
     auto dkdv = [&](float* a, float* b) {
         return two ? launch_gen_role<0, D, NP, DC, G2>(in, w, kb, a, b, BH, H, S, scale, causal, s)
                    : launch_gen_role<0, D, NP, DC, 1>(in, w, kb, a, b, BH, H, S, scale, causal, s);
@@ -2070,7 +2083,7 @@ int launch_gen_fwd(const AttnWs& w, const void* Q, const void* K, const void* V,
     const void* src[3] = {Q, K, V};
     const int rc = gen_planes<T, NP>(w, src, 3, pre, in, BH, S, D, rope_mode, theta, s);
     if (rc) return rc;
-    if (BH * ((S + 127) / 128) <= kGenSplitBlocks)
+    if (gen_two_groups(D, sizeof(T) == 4, false, BH * ((S + 127) / 128), S, causal))
         return launch_gen_fwd_g<T, D, NP, G2>(in, kb, O, LSE, BH, H, S, scale, causal, s);
     return launch_gen_fwd_g<T, D, NP, 1>(in, kb, O, LSE, BH, H, S, scale, causal, s);
 }
@@ -2079,14 +2092,20 @@ template <typename T, int NP>
 int gen_fwd_dispatch(const AttnWs& w, const void* Q, const void* K, const void* V, const float* kb,
                      void* O, float* LSE, int B, int H, int S, int D, float scale, int causal,
                      int rope_mode, float theta, hipStream_t s) {
+#define GN_GEN(DV)                                                                              \
+    case DV:                                                                                    \
+        return launch_gen_fwd<T, DV, NP>(w, Q, K, V, kb, O, LSE, B, H, S, scale, causal, rope_mode, theta, s);
     switch (D) {
-        case 32: return launch_gen_fwd<T, 32, NP>(w, Q, K, V, kb, O, LSE, B, H, S, scale, causal, rope_mode, theta, s);
-        case 64: return launch_gen_fwd<T, 64, NP>(w, Q, K, V, kb, O, LSE, B, H, S, scale, causal, rope_mode, theta, s);
-        case 96: return launch_gen_fwd<T, 96, NP>(w, Q, K, V, kb, O, LSE, B, H, S, scale, causal, rope_mode, theta, s);
-        case 128: return launch_gen_fwd<T, 128, NP>(w, Q, K, V, kb, O, LSE, B, H, S, scale, causal, rope_mode, theta, s);
-        case 192: return launch_gen_fwd<T, 192, NP>(w, Q, K, V, kb, O, LSE, B, H, S, scale, causal, rope_mode, theta, s);
-        case 256: return launch_gen_fwd<T, 256, NP>(w, Q, K, V, kb, O, LSE, B, H, S, scale, causal, rope_mode, theta, s);
+        GN_GEN(32)
+        GN_GEN(96)
+        GN_GEN(192)
+        GN_GEN(256)
     }
+    if constexpr (NP == 2) switch (D) {  // (bf16: the kernels above)
+        GN_GEN(64)
+        GN_GEN(128)
+    }
+#undef GN_GEN
     set_error("gn_attn_fwd: generic path has no D=%d", D);
     return GN_E_INVALID;
 }
@@ -2105,6 +2124,8 @@ int gen_bwd_dispatch(const AttnWs& w, const void* Q, const void* K, const void* 
         GN_GEN(96)
         GN_GEN(192)
         GN_GEN(256)
+    }
+    if constexpr (NP == 2) switch (D) {  // (bf16: the kernels above)
         GN_GEN(64)
         GN_GEN(128)
     }
@@ -2135,11 +2156,8 @@ int attn_bwd_impl(const void* Q, const void* K, const void* V, const void* O, co
             set_error("gn_attn_bwd: workspace %zu B < %zu B", ws_bytes, need);
             return GN_E_WORKSPACE;
         }
-        if (sizeof(T) == 4)
-            return gen_bwd_dispatch<T, 2>(w, Q, K, V, O, dO, LSE, mask, dQ, dK, dV, B, H, S, D, scale,
-                                          causal, rope_mode, theta, s);
-        return gen_bwd_dispatch<T, 1>(w, Q, K, V, O, dO, LSE, mask, dQ, dK, dV, B, H, S, D, scale,
-                                      causal, rope_mode, theta, s);
+        return gen_bwd_dispatch<T, sizeof(T) == 4 ? 2 : 1>(w, Q, K, V, O, dO, LSE, mask, dQ, dK, dV, B, H, S, D,
+                                                           scale, causal, rope_mode, theta, s);
     }
     AttnWs w;
     const size_t need = ws_layout(BH, S, D, sizeof(T), mfma_ok ? kWsMfma : kWsSimt, ws, &w);
