@@ -28,7 +28,7 @@ __global__ __launch_bounds__(512, 1) void gemm_stream(GemmDesc g) {
     constexpr int A_ELEMS = BM * BK, B_ELEMS = BN * BK, STAGE_B = (A_ELEMS + B_ELEMS) * 2;
     constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 32, FN = WN / 32, NM = FM * FN;
     constexpr int RA = TA ? 2 : 1, RB = TB ? 1 : 2, NR = FM * RA + FN * RB;
-    constexpr int NDA = BM / (8 * NW), NDB = BN / (8 * NW), ND = NDA + NDB;
+    constexpr int ND = (BM + BN) / (8 * NW);  // DMA instructions of a wave per k-tile
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const uint32_t lds0 = lds_addr(smem_raw);
 
@@ -52,47 +52,20 @@ __global__ __launch_bounds__(512, 1) void gemm_stream(GemmDesc g) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = (wave >> 1) & 1, wn = wave & 1, dw = wave & 3;
-    const int kt0 = (g.Ks[0] + BK - 1) / BK;
-    const int KT = kt0 + (g.nseg > 1 ? (g.Ks[1] + BK - 1) / BK : 0);
+    const int KT = (g.Ks[0] + BK - 1) / BK + (g.nseg > 1 ? (g.Ks[1] + BK - 1) / BK : 0);
     const int J = ntile * KT;  // k-tiles of the stream
 
     if (wave >= 4) {
         // producers: the compute waves' barriers, the DMA of k-tile j + STAGES after each
-        uint32_t voa[NDA], vob[NDB];
-        int pi = 0, pt = 0, m0, n0, oseg = -1;  // next k-tile to move
+        KFeed<TA, TB, BM, BN, NW> feed(g, dw);
+        int pi = 0, m0, n0;
         tile_at(0, m0, n0);
+        feed.start(m0, n0, 0);
         auto next = [&](int slot) __attribute__((always_inline)) {
-            const bool s1 = pt >= kt0;
-            const int k0 = (s1 ? pt - kt0 : pt) * BK, klim = s1 ? g.Ks[1] : g.Ks[0];
-            const bf16_t* A = g.A[s1];
-            const bf16_t* B = g.B[s1];
-            const int lda = g.lda[s1], ldb = g.ldb[s1];
-            const uint32_t base = lds0 + (uint32_t)(slot * STAGE_B);
-            if (k0 + BK > klim) {
-                stage_tail<BM, !TA, NW>(A, lda, m0, g.M, k0, klim, dw, base);
-                stage_tail<BN, TB, NW>(B, ldb, n0, g.N, k0, klim, dw, base + A_ELEMS * 2);
-            } else {
-                if (oseg != (int)s1) {
-                    oseg = s1;
-                    stage_offsets<BM, !TA, NW>(lda, m0, g.M, dw, voa);
-                    stage_offsets<BN, TB, NW>(ldb, n0, g.N, dw, vob);
-                }
-                const bf16_t* sa = stage_base<!TA>(A, lda, m0, k0);
-                const bf16_t* sb = stage_base<TB>(B, ldb, n0, k0);
-#pragma unroll
-                for (int q = 0; q < NDA; ++q) dma16s(sa, voa[q], base + 1024u * (uint32_t)(dw * NDA + q));
-#pragma unroll
-                for (int q = 0; q < NDB; ++q)
-                    dma16s(sb, vob[q], base + A_ELEMS * 2 + 1024u * (uint32_t)(dw * NDB + q));
-            }
-            if (++pt == KT) {
-                if (pi + 1 < ntile) {
-                    pt = 0;
-                    tile_at(++pi, m0, n0);
-                    oseg = -1;  // row and column clamps are the tile's
-                } else {
-                    pt = KT - 1;  // past the end: the last k-tile again
-                }
+            feed.issue(lds0 + (uint32_t)(slot * STAGE_B));
+            if (!feed.step() && pi + 1 < ntile) {  // past the end: the last k-tile again
+                tile_at(++pi, m0, n0);
+                feed.start(m0, n0, 0);
             }
         };
         static_for<STAGES>([&](auto S_) { next(decltype(S_)::value); });
