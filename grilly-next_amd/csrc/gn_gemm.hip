@@ -647,7 +647,8 @@ size_t weight_grad_ws_bytes(int M, int N, int Kin, int dtype) {
 // limited to what fits).
 int gemm_dispatch(const void* A0, const void* B0, int K0, const void* A1, const void* B1, int K1,
                   void* C, int M, int N, int transA, int transB, int dtype, int c_dtype,
-                  unsigned flags, hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0) {
+                  unsigned flags, hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0,
+                  bool beside = false) {
     GN_REQUIRE(M >= 0 && N >= 0 && K0 >= 0 && K1 >= 0, "gn_gemm: negative size");
     if (M == 0 || N == 0) return GN_OK;
     GN_REQUIRE(C, "gn_gemm: null C");
@@ -672,6 +673,7 @@ int gemm_dispatch(const void* A0, const void* B0, int K0, const void* A1, const 
     }
     d.M = M; d.N = N; d.C = C; d.C2 = C; d.Msplit = M; d.ldc = N;
     d.accumulate = acc ? 1 : 0;
+    d.beside = beside;
     if (ws && al16(ws)) {
         d.part = (float*)ws;
         d.part_cap = ws_bytes;
@@ -865,7 +867,7 @@ extern "C" int gn_linear_bwd_ws(const void* dY, const void* X, const void* W, vo
                          ws_bytes, sb.side() != s);
     if (rc == GN_OK && dX)  // dX[M x K] = dY[M x N] . W[N x K]
         rc = gemm_dispatch(dY, W, N, nullptr, nullptr, 0, dX, M, K, 0, 0, dtype, dtype, flags,
-                           sb.side(), dtype == GN_F32 ? ws : nullptr, ws_bytes);
+                           sb.side(), dtype == GN_F32 ? ws : nullptr, ws_bytes, sb.side() != s);
     const int jr = sb.join();
     return rc ? rc : jr;
 }
@@ -942,6 +944,7 @@ static int glu_proj_impl(const void* gu, const void* X, const void* Wg, const vo
         d.A[1] = (const bf16_t*)(g0 + (size_t)H * esz); d.lda[1] = 2 * H;
         d.B[1] = (const bf16_t*)Wu; d.ldb[1] = K; d.Ks[1] = H;
         d.M = M; d.N = K; d.C = dX; d.C2 = dX; d.Msplit = M; d.ldc = K; d.accumulate = acc;
+        d.beside = sb.side() != s;
         rc = gemm_run(d, 0, 0, dtype, dtype, sb.side());
     }
     const int jr = sb.join();
