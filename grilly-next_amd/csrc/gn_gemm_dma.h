@@ -90,6 +90,8 @@ int gemm_dma_f32_ta0(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_f32_ta1(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s);
 int gemm_dma_glu(const GemmDesc& g, int transA, int transB, hipStream_t s);
+// the time (us) gemm_dma_bf16's tiles are expected to take, for a choice between the kernels
+double gemm_stream_us(const GemmDesc& g);
 // fp32 C of an unbiased weight gradient (transA, plain epilogue) on streamed tiles, where it wins
 bool gemm_stream_f32_wins(const GemmDesc& g, int transA, int transB);
 int gemm_stream_f32(const GemmDesc& g, hipStream_t s);

@@ -272,6 +272,20 @@ int stream_blocks() {
     return std::max(8, cus / 8 * 8);
 }
 
+// Tile rows for g, and the time the product then takes (us, bf16 C): rounds of 256 x 128 or
+// 128 x 128 tiles, whichever need less.  A round of the small ones takes 0.6 of a round of the
+// large: 4.2 us + 0.29 per k-tile against 6.5 + 0.52 (up to 0.4 and 0.6 where a round fills the
+// chip).  Measured, 256 -> 128 rows: 4096 x 768 x 3072 (one round either way) 33 -> 24 us, 2048^3
+// 24.5 -> 20.2; 8192 x 768 x 3072 (one round against two) 39 -> 48, 2816 x 2304 x 768 14 -> 16.
+int choose_rows(const GemmDesc& g, int blocks, double* us) {
+    const long tn = (g.N + 127) / 128;
+    const long r256 = ((g.M + 255) / 256 * tn + blocks - 1) / blocks;
+    const long r128 = ((g.M + 127) / 128 * tn + blocks - 1) / blocks;
+    const bool small = 0.62 * (double)r128 < (double)r256;
+    *us = small ? (double)r128 * (4.2 + 0.29 * k_tiles(g)) : (double)r256 * (6.5 + 0.52 * k_tiles(g));
+    return small ? 128 : 256;
+}
+
 template <int BM>
 int launch_tile(const GemmDesc& g, int transA, int transB, int blocks, hipStream_t s) {
     if (!transA && !transB) return launch<false, false, BM>(g, blocks, s);
@@ -282,23 +296,28 @@ int launch_tile(const GemmDesc& g, int transA, int transB, int blocks, hipStream
 
 }  // namespace
 
-// 256 x 128 or 128 x 128 tiles, whichever needs less time for its rounds: a round of the small
-// ones takes 0.6 of a round of the large (a k-tile 0.42 against 0.67 us, fixed 4.5 against 7 us).
-// Measured, 256 -> 128 rows: 4096 x 768 x 3072 (one round either way) 33 -> 24 us, 2048^3 24.5 ->
-// 20.2; 8192 x 768 x 3072 (one round against two) 39 -> 48, 2816 x 2304 x 768 14 -> 16.
-int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s) {
-    const int cus = stream_blocks();
-    const long tn = (g.N + 127) / 128;
-    const long r256 = ((g.M + 255) / 256 * tn + cus - 1) / cus, r128 = ((g.M + 127) / 128 * tn + cus - 1) / cus;
-    return 0.62 * (double)r128 < (double)r256 ? launch_tile<128>(g, transA, transB, cus, s)
-                                              : launch_tile<256>(g, transA, transB, cus, s);
+double gemm_stream_us(const GemmDesc& g) {
+    double us;
+    choose_rows(g, stream_blocks(), &us);
+    return us;
 }
 
-// More than two rounds of 256 x 128 tiles, alone on the GPU.  Measured (us, a block per tile -> here, M x N x K
-// of dW): 11264 x 2048 x 4096 178 -> 159, x 2048 112 -> 91, x 300 55 -> 32; 32000 x 768 x 2001 120 -> 95;
+int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s) {
+    if (g.Msplit < g.M) {
+        set_error("gemm: a bf16 product has one destination");
+        return GN_E_INVALID;
+    }
+    const int blocks = stream_blocks();
+    double us;
+    return choose_rows(g, blocks, &us) == 128 ? launch_tile<128>(g, transA, transB, blocks, s)
+                                              : launch_tile<256>(g, transA, transB, blocks, s);
+}
+
+// More than two rounds of 256 x 128 tiles, alone on the GPU.  Measured (us, a block per tile -> here,
+// M x N x K of dW): 11264 x 2048 x 4096 180 -> 172, x 2048 112 -> 91; 32000 x 768 x 2001 120 -> 95;
 // 8192 x 8192 x 4096 555 -> 472; the least gain just above the line (10240 x 1792 x 4096, 560 tiles,
-// 153 -> 149).  Beside another product (an LM head's dX, 48 tiles over K = 32000) blocks that stay keep it
-// waiting: the pair's pass 522 -> 532, so there the core's blocks go on sharing the GPU.
+// 153 -> 149).  Beside another product (an LM head's dX, 48 tiles over K = 32000) the core's blocks go
+// on sharing the GPU: with blocks that stay the pair's pass was 522 -> 532.
 bool gemm_stream_f32_wins(const GemmDesc& g, int transA, int transB) {
     if (!transA || transB || g.bias || g.cbias || g.beside) return false;
     const long tiles = (long)((g.M + 255) / 256) * ((g.N + 127) / 128);

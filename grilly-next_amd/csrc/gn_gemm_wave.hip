@@ -220,25 +220,31 @@ int launch_plain(const GemmDesc& g, int ta, int tb, int shape, hipStream_t s) {
 
 }  // namespace
 
-// The tile that runs g fastest here, or -1 where the core's tiles do.  Time model, fitted to
+// The tile that runs g fastest here, or -1 where the large tiles do.  Time model, fitted to
 // MI355X sweeps of both over M from 1 to 4096 on the FFN and decoder products: a round of
 // blocks (one per CU) takes a fixed time and one step per four k-tiles; the steps are bound by
 // the LDS DMA (64 x 64: 64 KB in 0.7 us = 92 GB/s per CU), so a small tile pays where
-// the core's grid leaves CUs idle: its larger tiles move half the bytes per FLOP but take
-// 0.3-0.55 us per k-tile on however few CUs.  Measured (us, core -> here): 37 x 5632 x 2048
-// 13.9 -> 8.2, 37 x 2048 x 5632 28.0 -> 10.6, 300 x 2048 x 5632 33.8 -> 19.1, 1003 x 768 x 6144
-// 38.8 -> 22.3, dW 768 x 768 over 1003 rows 11.3 -> 8.2; level at 1003 x 2048 x 5632 and
-// 2001 x 768 x 6144; the core leads from there (2001 x 2048 x 5632 45.9 against 73.5).  The line is
-// drawn at 0.85 of the core's modelled time, where the two measured level.
+// the large ones leave CUs idle: they move half the bytes per FLOP but take 0.3-0.55 us per k-tile
+// on however few CUs.  The other side is the kernel that would run instead: bf16 C the streamed
+// tiles (gemm_stream_us), fp32 C and the GLU epilogue the core's.
+// Measured (us, replayed; streamed tiles -> here): 64 x 5632 x 2048 13.2 -> 7.8, 64 x 2048 x 5632
+// 28.9 -> 10.3, 384 x 2048 x 5632 33.4 -> 20.0, 1003 x 768 x 6144 40.9 -> 24.6, an LM head's dX 16 x 768 x
+// 32000 142 -> 61, 1003 rows 175 -> 98; the streamed tiles lead at 200 x 5632 x 2048 (13.7 against 17.1),
+// 768 x 2048 x 5632 (34.4 / 36.5), 1536 x 768 x 6144 (38.5 / 39.3) and 2001 x 768 x 32000 (level alone, 279
+// against 342 beside its weight gradient).  fp32 C, core -> here: dW 768 x 768 over 512 rows 8.6 -> 5.8,
+// over 4096 23.7 -> 17.6.  Of 240 bf16 products in that sweep the lines drawn (0.95 of the streamed
+// time, 0.85 of the core's) give each the faster kernel.
 int gemm_wave_shape(const GemmDesc& g, int transA, int transB, int c_dtype) {
-    // a very long k loop (an LM head's dX, 2001 x 768 x 32000) is level alone, 171 against 176 us,
-    // and slower beside its weight gradient, to which the core's part-filled grid leaves CUs
-    if (k_tiles(g) > 256) return -1;
     const bool ta = transA != 0;
     const size_t c_bytes = g.epi == 1 || c_dtype != GN_F32 ? 2 : 4;
-    const TileChoice tc = choose_tile(g, ta, c_bytes, g.epi);
-    if (tc.m_first > 0) return -1;
-    double best = 0.85 * tile_cost(g, ta, c_bytes, g.epi, tc.shape, tc.ksplit, tc.ksplit > 2);
+    double best;
+    if (g.epi == 0 && c_bytes == 2) {
+        best = 0.95 * gemm_stream_us(g);
+    } else {
+        const TileChoice tc = choose_tile(g, ta, c_bytes, g.epi);
+        if (tc.m_first > 0) return -1;
+        best = 0.85 * tile_cost(g, ta, c_bytes, g.epi, tc.shape, tc.ksplit, tc.ksplit > 2);
+    }
     static constexpr int bm[4] = {64, 64, 32, 32}, bn[4] = {64, 32, 64, 32};
     static constexpr double fixed[4] = {3.2, 1.8, 1.8, 1.6}, step[4] = {0.70, 0.52, 0.52, 0.34};
     const int steps = (k_tiles(g) + 3) / 4;

@@ -36,3 +36,13 @@ def test_input_gradient_of_several_rounds_beside_its_weight_gradient(gn, M, N, K
     torch.cuda.synchronize()
     assert err(dX, dY.double() @ W.double()) < 2.0 ** -8
     assert err(dW, dY.double().t().contiguous() @ X.double()) < 2e-5
+
+
+@pytest.mark.parametrize("K", [16384, 16392, 20008])
+@pytest.mark.parametrize("M,N", [(16, 768), (65, 264), (300, 136)])
+def test_few_rows_over_a_long_k(gn, M, N, K):
+    """An LM head's dX on few tokens: K (the vocabulary) shared by a block's waves at any length."""
+    A, B = rand(4, M, K), rand(5, K, N)
+    assert err(gn.gemm(A, B, out_dtype=BF), A.double() @ B.double()) < 2.0 ** -8
+    dW = gn.gemm(rand(6, K, 136), rand(7, K, 72), transA=True, out_dtype=torch.float32)
+    assert err(dW, rand(6, K, 136).double().t().contiguous() @ rand(7, K, 72).double()) < 2e-5
