@@ -594,7 +594,7 @@ int weight_grad(const void* dY, int ldy, const void* X, int ldx, int M, int N, i
     // end to end (12-layer decoder, one box, interleaved runs) fusing every bias beat both the
     // two-pass column sum everywhere (9.73 vs 10.01 ms per step) and fusing only GEMMs under
     // 48 us (9.94 ms): the two extra launches per bias cost more than their kernel time.
-    if (db && dtype == GN_BF16 && gemm_dma_applicable(d, 1, 0)) {
+    if (db && dtype == GN_BF16 && gemm_dma_applicable(d, 1, 0) && !gemm_stream_sums_apart(d)) {
         d.bias = db;
         d.bias2 = db2 ? db2 : db + Msplit;
         return gemm_dma_launch(d, 1, 0, GN_F32, s);

@@ -95,6 +95,9 @@ double gemm_stream_us(const GemmDesc& g);
 // fp32 C of an unbiased weight gradient (transA, plain epilogue) on streamed tiles, where it wins
 bool gemm_stream_f32_wins(const GemmDesc& g, int transA, int transB);
 int gemm_stream_f32(const GemmDesc& g, hipStream_t s);
+// whether a biased weight gradient (g without its bias) is better off with its row sums taken apart,
+// the product then on streamed tiles
+bool gemm_stream_sums_apart(const GemmDesc& g);
 // Small tiles with K split over a block's waves (gn_gemm_wave.hip), for products that the core's
 // tiles would spread over too few compute units: the tile shape to run g on, or -1 (the core).
 int gemm_wave_shape(const GemmDesc& g, int transA, int transB, int c_dtype);

@@ -313,19 +313,37 @@ int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s) {
                                               : launch_tile<256>(g, transA, transB, blocks, s);
 }
 
-// More than two rounds of 256 x 128 tiles, alone on the GPU.  Measured (us, a block per tile -> here,
+// Up to 1024 rows of dY and X, where a dW tile is mostly its store: this one leaves as whole row
+// segments, the core's, staged per wave, in half the speed (us, register-staged 128 x 128 tiles -> core
+// -> here, M x N x K of dW): 2048 x 2048 x 8 8.1 -> 14.9 -> 8.2, x 200 11.0 -> 14.4 -> 9.2, x 1003
+// 25 -> 20.0 -> 14.6; 5632 x 2048 x 200 21.2 -> 31.0 -> 16.7; 4096 x 4096 x 8 16.4 -> 33.2 -> 17.2.
+constexpr int kShortK = 16;  // k-tiles
+
+// Or more than two rounds of 256 x 128 tiles, alone on the GPU.  Measured (us, a block per tile -> here,
 // M x N x K of dW): 11264 x 2048 x 4096 180 -> 172, x 2048 112 -> 91; 32000 x 768 x 2001 120 -> 95;
 // 8192 x 8192 x 4096 555 -> 472; the least gain just above the line (10240 x 1792 x 4096, 560 tiles,
 // 153 -> 149).  Beside another product (an LM head's dX, 48 tiles over K = 32000) the core's blocks go
 // on sharing the GPU: with blocks that stay the pair's pass was 522 -> 532.
 bool gemm_stream_f32_wins(const GemmDesc& g, int transA, int transB) {
-    if (!transA || transB || g.bias || g.cbias || g.beside) return false;
+    if (!transA || transB || g.bias || g.cbias) return false;
     const long tiles = (long)((g.M + 255) / 256) * ((g.N + 127) / 128);
-    return tiles > 2L * stream_blocks();
+    return k_tiles(g) <= kShortK || (!g.beside && tiles > 2L * stream_blocks());
+}
+
+// Over a round of such tiles the column sums' own launch (one, ~5 us, up to these 1024 rows) costs less
+// than the core's store: backward with db of 200 x 5632 x 2048 (replayed) 42.7 with the register-staged
+// tiles -> 53.4 on the core -> 41 here; of 200 x 2048 x 2048, 128 tiles, 23.0 with the core's fused sums,
+// which stays.
+bool gemm_stream_sums_apart(const GemmDesc& g) {
+    const long tiles = (long)((g.M + 255) / 256) * ((g.N + 127) / 128);
+    return k_tiles(g) <= kShortK && tiles > stream_blocks() && gemm_stream_f32_wins(g, 1, 0);
 }
 
 int gemm_stream_f32(const GemmDesc& g, hipStream_t s) {
-    return launch<true, false, 256, float>(g, stream_blocks(), s);
+    const int blocks = stream_blocks();
+    double us;
+    if (k_tiles(g) <= kShortK && choose_rows(g, blocks, &us) == 128) return launch<true, false, 128, float>(g, blocks, s);
+    return launch<true, false, 256, float>(g, blocks, s);
 }
 
 }  // namespace gn

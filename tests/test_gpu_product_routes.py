@@ -46,3 +46,23 @@ def test_few_rows_over_a_long_k(gn, M, N, K):
     assert err(gn.gemm(A, B, out_dtype=BF), A.double() @ B.double()) < 2.0 ** -8
     dW = gn.gemm(rand(6, K, 136), rand(7, K, 72), transA=True, out_dtype=torch.float32)
     assert err(dW, rand(6, K, 136).double().t().contiguous() @ rand(7, K, 72).double()) < 2e-5
+
+
+@pytest.mark.parametrize("T", [1, 8, 63, 64, 65, 200, 1023, 1024, 1025])
+@pytest.mark.parametrize("N,K", [(136, 72), (2056, 1040), (5640, 2056)])
+@pytest.mark.parametrize("db", [False, True])
+def test_weight_gradient_of_few_rows(gn, T, N, K, db):
+    """Either side of 16 k-tiles (1024 rows), with ragged tiles, at one round of them and above, where
+    the column sums of dY are taken apart; stored, then added to what is there."""
+    dY, X, W = rand(8, T, N, std=0.01), rand(9, T, K), rand(10, N, K, std=0.02)
+    ref, sums = dY.double().t().contiguous() @ X.double(), dY.double().sum(0)
+    _, dW, dB = gn.linear_bwd(dY, X, W, need_dx=False, need_db=db)
+    assert err(dW, ref) < 2e-5 and (not db or err(dB, sums) < 2e-5)
+    gn.linear_bwd(dY, X, W, need_dx=False, need_db=db, dW=dW, db=dB, accumulate=True)
+    assert err(dW, 2 * ref) < 2e-5 and (not db or err(dB, 2 * sums) < 2e-5)
+
+
+def test_weight_gradient_of_few_rows_over_two_rounds_of_tiles(gn):
+    dY, X = rand(11, 8, 8192), rand(12, 8, 4096)
+    dW = gn.gemm(dY, X, transA=True, out_dtype=torch.float32)
+    assert err(dW, dY.double().t().contiguous() @ X.double()) < 2e-5
