@@ -232,7 +232,7 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_mfma(GemmDesc g) {
 constexpr int kSmallMaxK = 128;
 constexpr int64_t kSmallMaxMac = (int64_t)1 << 24;
 
-template <typename TI, typename CT, bool TA, bool TB>
+template <typename TI, typename CT, bool TA, bool TB, bool FB = false>
 __global__ __launch_bounds__(256) void gemm_small(GemmDesc g) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (int64_t)g.M * g.N) return;
@@ -249,6 +249,7 @@ __global__ __launch_bounds__(256) void gemm_small(GemmDesc g) {
             acc = fmaf(a, b, acc);
         }
     }
+    if constexpr (FB) acc += g.fbias[n];
     gemm_store<CT, 0>(g, m, n, acc);
 }
 
@@ -261,7 +262,8 @@ inline bool small_applicable(const GemmDesc& d) {
 template <typename TI, typename CT>
 int launch_small(const GemmDesc& g, int ta, int tb, hipStream_t s) {
     const unsigned grid = (unsigned)(((int64_t)g.M * g.N + 255) / 256);
-    if (!ta && !tb) gemm_small<TI, CT, false, false><<<grid, 256, 0, s>>>(g);
+    if (g.fbias) gemm_small<TI, CT, false, true, true><<<grid, 256, 0, s>>>(g);
+    else if (!ta && !tb) gemm_small<TI, CT, false, false><<<grid, 256, 0, s>>>(g);
     else if (!ta && tb) gemm_small<TI, CT, false, true><<<grid, 256, 0, s>>>(g);
     else if (ta && !tb) gemm_small<TI, CT, true, false><<<grid, 256, 0, s>>>(g);
     else gemm_small<TI, CT, true, true><<<grid, 256, 0, s>>>(g);
@@ -526,8 +528,8 @@ int gemm_run(const GemmDesc& d, int transA, int transB, int dtype, int c_dtype, 
         set_error("gemm: fused row sums need the LDS-DMA core (bf16 operands, fp32 C)");
         return GN_E_INVALID;
     }
-    if (d.fbias && !(dtype == GN_F32 && !d.accumulate)) {
-        set_error("gemm: the fp32 column bias goes with fp32 operands, overwriting C");
+    if (d.fbias && !(dtype == GN_F32 && !transA && transB && !d.accumulate)) {
+        set_error("gemm: the fp32 column bias goes with a forward Linear's fp32 product, overwriting C");
         return GN_E_INVALID;
     }
     if (d.cbias && !(dtype == GN_BF16 && d.epi == 0 && gemm_dma_applicable(d, transA, transB))) {

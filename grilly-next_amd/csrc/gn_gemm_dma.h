@@ -44,10 +44,6 @@ struct GemmDesc {
     // column bias of the plain epilogue (a forward Linear's b): C[m][n] = acc + cbias[n],
     // bf16, LDS-DMA core only, no split-K; nullptr: none
     const bf16_t* cbias;
-    // the same for an fp32 product (fp32 operands and C, overwritten); nullptr: none
-    const float* fbias;
-    // another product shares the GPU with this one (a call's side-by-side pair)
-    bool beside;
     // split-K through a workspace (plain fp32 epilogue, ksplit >= 3): split y stores its
     // partial tile at part + y*M*N (row-major, pitch N) and, with a bias, its row sums at
     // part + ksplit*M*N + y*M; split_reduce then adds the splits in index order into C and
@@ -55,6 +51,11 @@ struct GemmDesc {
     // available at part (0: no workspace; splits of two then add into C with atomics)
     float* part;
     size_t part_cap;
+    // the column bias of an fp32 product (a forward Linear's: A, op(B) untransposed and transposed,
+    // C overwritten), no split-K; nullptr: none
+    const float* fbias;
+    // another product shares the GPU with this one (a call's side-by-side pair)
+    bool beside;
 };
 
 // Store one accumulated element (m, n) according to the descriptor's epilogue.
@@ -126,7 +127,6 @@ __device__ __forceinline__ void gemm_store(const GemmDesc& g, int m, int n, floa
     if constexpr (EPI == 0) {
         CT* C = reinterpret_cast<CT*>(m < g.Msplit ? g.C : g.C2);
         const size_t idx = (size_t)(m < g.Msplit ? m : m - g.Msplit) * g.ldc + n;
-        if (g.fbias) v += g.fbias[n];
         io<CT>::st(C, idx, g.accumulate ? v + io<CT>::ld(C, idx) : v);
     } else {
         const size_t gi = (size_t)m * g.ldg + n;
@@ -146,17 +146,20 @@ __device__ __forceinline__ void gemm_store(const GemmDesc& g, int m, int n, floa
 
 // Epilogue of one 32x32 MFMA accumulator tile (lane layout: col = lane%32, row =
 // 8(r/4) + 4(lane/32) + r%4) at (m0, n0).  For the GLU epilogue all 32 gate/up loads of
-// the tile are issued before any store, so their latencies overlap.
-template <typename CT, int EPI, typename ACC>
+// the tile are issued before any store, so their latencies overlap.  FB: with the fp32 column bias
+// (the kernels of fp32 operands).
+template <typename CT, int EPI, bool FB = false, typename ACC>
 __device__ __forceinline__ void gemm_store_tile(const GemmDesc& g, int m0, int n0, const ACC& a) {
     const int lane = threadIdx.x & 63;
     const int n = n0 + (lane & 31), rq = (lane >> 5) * 4;
     if (n >= g.N) return;
     if constexpr (EPI == 0) {
+        float b = 0.f;
+        if constexpr (FB) b = g.fbias[n];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = m0 + 8 * (r >> 2) + rq + (r & 3);
-            if (m < g.M) gemm_store<CT, 0>(g, m, n, a[r]);
+            if (m < g.M) gemm_store<CT, 0>(g, m, n, FB ? a[r] + b : a[r]);
         }
     } else {
         const bf16_t* __restrict__ gp = g.gate;

@@ -66,3 +66,21 @@ def test_weight_gradient_of_few_rows_over_two_rounds_of_tiles(gn):
     dY, X = rand(11, 8, 8192), rand(12, 8, 4096)
     dW = gn.gemm(dY, X, transA=True, out_dtype=torch.float32)
     assert err(dW, dY.double().t().contiguous() @ X.double()) < 2e-5
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (5, 33, 17), (64, 10, 32),                # scalar tiles
+    (512, 10, 256), (70, 21, 300),            # MFMA chain, 16- and 32-wide
+    (128, 256, 512), (130, 100, 264),         # 32 x 32 tiles of six products
+    (2048, 1024, 1024), (2050, 1028, 1000),   # 128 x 128
+    (64, 40000, 512), (33, 40004, 260)])      # 64 x 256
+@pytest.mark.parametrize("shift", [0, 1])
+def test_biased_fp32_forward_on_every_kernel(gn, M, N, K, shift):
+    """The column bias added by the product's own kernel, aligned and not, and the product without it.
+    fp32 sums: sqrt(K) 2^-24 rms of an entry, five times that over the largest of 2e6 entries, which is
+    itself five times the rms: < 2e-6 of the largest at K <= 1024."""
+    X, W = rand(13, M, K, dtype=torch.float32), rand(14, N, K, dtype=torch.float32)
+    b = rand(15, N + 1, dtype=torch.float32)[shift:shift + N]
+    ref = X.double() @ W.double().t()
+    assert err(gn.linear_fwd(X, W), ref) < 2e-6
+    assert err(gn.linear_fwd(X, W, b), ref + b.double()) < 2e-6
