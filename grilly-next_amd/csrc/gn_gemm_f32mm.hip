@@ -250,8 +250,10 @@ __global__ __launch_bounds__(64) void gemm_f32x6t(GemmDesc g) {
 
 }  // namespace
 
-// Time model (us) fitted to MI355X sweeps: gemm_f32x6 takes 0.72 us per 16-k stage on however few
-// blocks and slows from ~340 blocks on, a 32 x 32 tile 0.42 us per stage up to ~800 tiles.
+// Time model (us) fitted to MI355X sweeps (251 products, K from 4 to 3072): gemm_f32x6 takes 0.63 us per
+// 16-k stage on however few blocks and slows from ~220 blocks on, a 32 x 32 tile 0.44 us per stage up to
+// ~900 tiles, and a tile's launch and store 1.4 ns (a short K of many tiles is gemm_f32x6's:
+// 1536 x 1536 x 16 6.4 against 8.1, 3072 x 3072 x 16 10.6 against 17.5).
 // Measured (gemm_f32x6 -> here): 64 x 256 x 784 (one block) 40 -> 20, 1000 x 512 x 784 37.6 -> 21.7,
 // 512 x 1536 x 1536 73 -> 41, 200 x 4000 x 1000 46 -> 28; gemm_f32x6 keeps 2048 x 1024 x 1024 (50 against 63) and
 // 64 x 163840 x 1536 (285 against 545).  Split-K products stay with gemm_f32x6 too (their planes
@@ -262,8 +264,8 @@ bool gemm_f32x6t_wins(const GemmDesc& g) {
     gemm_f32_grid(g, blocks, stages, ks);
     if (ks > 1) return false;
     const double tiles = (double)((g.M + 31) / 32) * ((g.N + 31) / 32);
-    const double x6 = 4.0 + 0.72 * stages * std::max(1.0, (double)blocks / 340.0);
-    return 2.0 + 0.42 * stages * std::max(1.0, tiles / 800.0) < 0.9 * x6;
+    const double x6 = 5.0 + 0.009 * (double)blocks + 0.63 * stages * std::max(1.0, (double)blocks / 220.0);
+    return 4.2 + 0.0014 * tiles + 0.44 * stages * std::max(1.0, tiles / 900.0) < x6;
 }
 
 int gemm_f32x6t_launch(const GemmDesc& g, int transA, int transB, hipStream_t s) {

@@ -84,3 +84,14 @@ def test_biased_fp32_forward_on_every_kernel(gn, M, N, K, shift):
     ref = X.double() @ W.double().t()
     assert err(gn.linear_fwd(X, W), ref) < 2e-6
     assert err(gn.linear_fwd(X, W, b), ref + b.double()) < 2e-6
+
+
+@pytest.mark.parametrize("M,N,K", [(1536, 1536, 16), (1540, 1532, 20), (768, 768, 16), (3072, 3072, 16),
+                                   (1024, 1024, 64), (516, 772, 36)])
+@pytest.mark.parametrize("tA,tB", [(False, True), (True, False)])
+def test_fp32_product_of_short_k(gn, M, N, K, tA, tB):
+    """Either side of the line between 32 x 32 and larger tiles, where K is a few 16-wide stages."""
+    A = rand(16, *((K, M) if tA else (M, K)), dtype=torch.float32)
+    B = rand(17, *((N, K) if tB else (K, N)), dtype=torch.float32)
+    ref = (A.double().t() if tA else A.double()) @ (B.double().t() if tB else B.double())
+    assert err(gn.gemm(A, B, transA=tA, transB=tB), ref) < 2e-6
