@@ -160,33 +160,49 @@ __device__ __forceinline__ float gumbel(uint64_t seed, uint64_t idx) {
     return -logf(-logf(u));
 }
 
-// one block per row, 16 waves: a row's K x D predictions are read once, up to 16 branches'
-// loads in flight per thread, so a single row (batch 1) is not held to one wave's round trips
+// y z = +-z: the hinge terms gamma - y z of four elements
+__device__ __forceinline__ float hinge_sum4(const float4& z, uint32_t nib, float gamma) {
+    return fmaxf(gamma - sgn(z.x, nib), 0.f) + fmaxf(gamma - sgn(z.y, nib >> 1), 0.f) +
+           fmaxf(gamma - sgn(z.z, nib >> 2), 0.f) + fmaxf(gamma - sgn(z.w, nib >> 3), 0.f);
+}
+
+// one block per row, 16 waves: a row's K x D predictions are read once (without ONE the winner's D
+// twice), up to 16 branches' loads in flight per thread, so a single row (batch 1) is not held to one wave's round trips
 constexpr int kSurThreads = 1024, kSurWaves = kSurThreads / 64;
 
 // KG: branches per pass over D.  Four (K <= 4) keep the kernel at 64 registers, two blocks per CU.
-// Every branch's hinge sum is formed beside its dot product, so the winner's row is not read
+// ONE: every branch's hinge sum is formed beside its dot product, so the winner's row is not read
 // again.  8192 rows x 4 x 10240: 349 -> 200 us (1.34 GB read once; the second read of the winning
-// quarter and the single resident block were the rest).
-template <int KG>
+// quarter and the single resident block were the rest).  Eight at a time (K > 4) the same, 1024 rows
+// x 8 x 10240 76 -> 58 us, x 16 131 -> 112 (sixteen at a time with their hinges: 128).  More than eight
+// over at most a block per CU are one block's chain of loads and sums: sixteen go out together and the
+// winner's row is read again, 1 x 16 x 10240 15.9 us (hinges beside 17.6), 256 x 32 x 1024 21.0 (23.8;
+// eight at a time 22.4).
+template <int KG, bool ONE>
 __global__ __launch_bounds__(kSurThreads, KG <= 4 ? 8 : 4) void surrogate_fwd_rows(
     const float* __restrict__ preds, const uint32_t* __restrict__ bits, float* __restrict__ dots,
     uint32_t* __restrict__ results, float* __restrict__ weights, float* __restrict__ loss,
     int Bn, int K, int D, int words, float gamma, float delta, float lambda_c, float temperature,
     uint64_t seed, uint64_t counter, int noise) {
-    __shared__ float sd[kSurrogateMaxK], sadj[kSurrogateMaxK], shinge[kSurrogateMaxK];
+    __shared__ float sd[kSurrogateMaxK], sadj[kSurrogateMaxK], shinge[ONE ? kSurrogateMaxK : 1];
+    __shared__ float sh[kSurWaves];
+    __shared__ int swin;
+    __shared__ float sdw, sdr;
     const int b = blockIdx.x, t = threadIdx.x;
     const uint32_t* yb = bits + (size_t)b * words;
     const int nc = D >> 2;  // D % 32 == 0
     // the branches' dot products in groups of KG: a thread's loads for all branches of a group
     // go out together (one memory round trip per chunk of D, not one per branch), each branch
     // then reduced as block_sum does (wave sum, the wave sums added in order from zero)
-    __shared__ float shk[KG][kSurWaves], shh[KG][kSurWaves];
+    __shared__ float shk[KG][kSurWaves], shh[ONE ? KG : 1][kSurWaves];
     const int wv = t >> 6, ln = t & 63;
     for (int k0 = 0; k0 < K; k0 += KG) {
-        float s[KG], h[KG];
+        float s[KG], h[ONE ? KG : 1];
 #pragma unroll
-        for (int j = 0; j < KG; ++j) s[j] = h[j] = 0.f;
+        for (int j = 0; j < KG; ++j) {
+            s[j] = 0.f;
+            if constexpr (ONE) h[j] = 0.f;
+        }
         for (int c = t; c < nc; c += kSurThreads) {
             const uint32_t nib = yb[c >> 3] >> (4 * (c & 7));
             float4 w[KG];
@@ -197,30 +213,31 @@ __global__ __launch_bounds__(kSurThreads, KG <= 4 ? 8 : 4) void surrogate_fwd_ro
             for (int j = 0; j < KG; ++j)
                 if (k0 + j < K) {
                     s[j] += signed_sum4(w[j], nib);
-                    // y z = +-z: the hinge term gamma - y z, one per element
-                    h[j] += fmaxf(gamma - sgn(w[j].x, nib), 0.f) + fmaxf(gamma - sgn(w[j].y, nib >> 1), 0.f) +
-                            fmaxf(gamma - sgn(w[j].z, nib >> 2), 0.f) + fmaxf(gamma - sgn(w[j].w, nib >> 3), 0.f);
+                    if constexpr (ONE) h[j] += hinge_sum4(w[j], nib, gamma);
                 }
         }
 #pragma unroll
         for (int j = 0; j < KG; ++j) {
             if (k0 + j >= K) break;
-            const float v = wave_sum(s[j]), u = wave_sum(h[j]);
-            if (ln == 0) {
-                shk[j][wv] = v;
-                shh[j][wv] = u;
+            const float v = wave_sum(s[j]);
+            if (ln == 0) shk[j][wv] = v;
+            if constexpr (ONE) {
+                const float u = wave_sum(h[j]);
+                if (ln == 0) shh[j][wv] = u;
             }
         }
         __syncthreads();
         if (t < KG && k0 + t < K) {
-            float tt = 0.f, hh = 0.f;
+            float tt = 0.f;
 #pragma unroll
-            for (int i = 0; i < kSurWaves; ++i) {
-                tt += shk[t][i];
-                hh += shh[t][i];
-            }
+            for (int i = 0; i < kSurWaves; ++i) tt += shk[t][i];
             sd[k0 + t] = tt;
-            shinge[k0 + t] = hh;
+            if constexpr (ONE) {
+                float hh = 0.f;
+#pragma unroll
+                for (int i = 0; i < kSurWaves; ++i) hh += shh[t][i];
+                shinge[k0 + t] = hh;
+            }
         }
         __syncthreads();
     }
@@ -255,7 +272,22 @@ __global__ __launch_bounds__(kSurThreads, KG <= 4 ? 8 : 4) void surrogate_fwd_ro
         results[(size_t)b * 4 + 1] = (uint32_t)k2;
         results[(size_t)b * 4 + 2] = __float_as_uint(sd[k1]);
         results[(size_t)b * 4 + 3] = __float_as_uint(sd[k2]);
-        loss[b] = shinge[k1] / (float)D + lambda_c * fmaxf(0.f, delta - (sd[k1] - sd[k2]));
+        if constexpr (ONE) {
+            loss[b] = shinge[k1] / (float)D + lambda_c * fmaxf(0.f, delta - (sd[k1] - sd[k2]));
+        } else {
+            swin = k1;
+            sdw = sd[k1];
+            sdr = sd[k2];
+        }
+    }
+    if constexpr (!ONE) {
+        __syncthreads();
+        const float* pw = preds + ((size_t)b * K + swin) * D;
+        float h = 0.f;
+        for (int c = t; c < nc; c += kSurThreads)
+            h += hinge_sum4(*reinterpret_cast<const float4*>(pw + 4 * c), yb[c >> 3] >> (4 * (c & 7)), gamma);
+        h = block_sum<kSurWaves>(h, sh);
+        if (t == 0) loss[b] = h / (float)D + lambda_c * fmaxf(0.f, delta - (sdw - sdr));
     }
 }
 
@@ -358,12 +390,11 @@ extern "C" int gn_vsa_surrogate_fwd(const float* preds, const uint32_t* bits, fl
     GN_REQUIRE(temperature > 0.f, "gn_vsa_surrogate_fwd: temperature must be > 0");
     hipStream_t s = as_stream(stream);
     const int noise = (flags & GN_NO_GUMBEL) ? 0 : 1;
-    if (K <= 4)
-        surrogate_fwd_rows<4><<<Bn, kSurThreads, 0, s>>>(preds, bits, dots, results, weights, loss, Bn, K, D, words,
-                                                         gamma, delta, lambda_c, temperature, seed, counter, noise);
-    else
-        surrogate_fwd_rows<16><<<Bn, kSurThreads, 0, s>>>(preds, bits, dots, results, weights, loss, Bn, K, D, words,
-                                                          gamma, delta, lambda_c, temperature, seed, counter, noise);
+    const auto rows = K <= 4                ? surrogate_fwd_rows<4, true>
+                      : K <= 8 || Bn > 256 ? surrogate_fwd_rows<8, true>
+                                           : surrogate_fwd_rows<16, false>;
+    rows<<<Bn, kSurThreads, 0, s>>>(preds, bits, dots, results, weights, loss, Bn, K, D, words, gamma, delta, lambda_c,
+                                    temperature, seed, counter, noise);
     GN_LAUNCH_CHECK("gn_vsa_surrogate_fwd");
     return GN_OK;
 }

@@ -103,6 +103,24 @@ def test_vsa_surrogate_fwd(env, Bn, K, D, noise):
     assert rel_err(loss.cpu().numpy(), l2) < FP32_TOL
 
 
+@pytest.mark.parametrize("K", [4, 5, 8, 9, 16, 17, 33])
+@pytest.mark.parametrize("Bn,D", [(1, 4128), (256, 96), (257, 96)])
+def test_vsa_surrogate_fwd_branches_and_rows(env, Bn, K, D):
+    """Every grouping of the branches, on either side of the lines that choose it, and a D over one
+    pass of the block's threads."""
+    gc, gb, gn, dev = env
+    rng = np.random.RandomState(11 + K)
+    bits = bits_of(rng, Bn, D // 32)
+    preds = rng.standard_normal((Bn, K, D)).astype(np.float32) * 0.5
+    dots, res, w, loss = gn.vsa_surrogate_fwd(torch.from_numpy(preds).cuda(), dev_bits(bits), noise=False)
+    dots, res = dots.cpu().numpy(), res.cpu().numpy().view(np.uint32)
+    assert rel_err(dots, oracle.vsa_dots(preds, bits)) < FP32_TOL
+    res_o, w_o = oracle.vsa_select(dots, 1.0, 0, 0, False)
+    np.testing.assert_array_equal(res, res_o)
+    assert rel_err(w.cpu().numpy(), w_o) < 1e-5
+    assert rel_err(loss.cpu().numpy(), oracle.vsa_surrogate_loss(preds, bits, res)) < FP32_TOL
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1536, 768), (2, 777, 1536), (5, 300, 64), (8, 640, 1024),
                                    (1, 10, 256), (4, 4096, 2048), (1, 999, 4096), (1, 5003, 1540)])
 def test_linear_fp32_skinny(env, M, N, K):
