@@ -704,15 +704,16 @@ def _opt_params(entries):
         n = W.numel()
         get = e.get
         lp = get("W_bf16")
-        ptrs = [_addr(W)]
+        ts = [W]
         for key in ("grad", "state0", "state1", "recalled"):
             x = get(key)
             if x is not None and not isinstance(x, int) and (x.dtype != f32 or x.numel() != n):
                 raise GnError(f"optimizer tensor {i}: {key} must be float32 with {n} elements")
-            ptrs.append(_addr(x))
+            ts.append(x)
         if lp is not None and (lp.numel() != n or lp.dtype != torch.bfloat16):
             raise GnError(f"optimizer tensor {i}: W_bf16 must be bfloat16 with {n} elements")
-        arr[i] = (*ptrs, _addr(lp), n)
+        e["grad"], e["state0"]  # KeyError: neither may be left out
+        arr[i] = (*map(_addr, ts), _addr(lp), n)
     return arr
 
 

@@ -161,3 +161,13 @@ def test_attention_row_strides_bounded_without_gpu():
             64, 64, big, 128, 384, 0.125, 1, 0, 1e4, 4, p(1 << 16), 1 << 24, None)
     assert lib.gn_attn_bwd_bshd(*args) == -1
     assert "below 2^24" in gn_bwd.last_error()
+
+
+@pytest.mark.parametrize("missing", ["grad", "state0"])
+def test_optimizer_entry_without_gradient_or_state_is_refused(missing):
+    """A key left out is an error by its name, not a null pointer handed to the kernels."""
+    import gn_bwd
+    import torch
+    e = {k: torch.zeros(4) for k in ("W", "grad", "state0", "state1") if k != missing}
+    with pytest.raises(KeyError, match=missing):
+        gn_bwd._opt_params([e])
