@@ -18,7 +18,9 @@
 // operand), so neither is ever written to LDS.  Two kernels (7 tile products instead of 5)
 // keep the dQ reduction free of atomics and deterministic.  The epilogues stage each
 // wave's rows in LDS and apply the inverse rotation from a cos/sin table.
-// A SIMT path (any D <= 256, fp32 or bf16) serves other shapes and the fp32 dtype.
+// fp32, and bf16 of D = 32, 96, 192 or 256, take the generic matrix-core path (attn_fwd_gen,
+// attn_bwd_gen: fp32 operands as bf16 pieces); a SIMT path (any D <= 256) the rest: other D, and
+// views that are not 16-byte aligned.
 //
 // Key-padding mask (flash-attention2.glsl:150-154, flash-attention2-rope.glsl:201-205: the
 // score of key k in batch b gets (mask[b S + k] - 1) 1e9): a pre-pass turns the mask into a

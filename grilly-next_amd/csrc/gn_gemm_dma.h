@@ -42,7 +42,7 @@ struct GemmDesc {
     float* bias;
     float* bias2;
     // column bias of the plain epilogue (a forward Linear's b): C[m][n] = acc + cbias[n],
-    // bf16, LDS-DMA core only, no split-K; nullptr: none
+    // bf16, where gemm_dma_applicable, no split-K; nullptr: none
     const bf16_t* cbias;
     // split-K through a workspace (plain fp32 epilogue, ksplit >= 3): split y stores its
     // partial tile at part + y*M*N (row-major, pitch N) and, with a bias, its row sums at
@@ -90,7 +90,7 @@ int gemm_dma_launch(const GemmDesc& g, int transA, int transB, int c_dtype, hipS
 int gemm_dma_f32_ta0(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_f32_ta1(const GemmDesc& g, int transB, hipStream_t s);
 int gemm_dma_bf16(const GemmDesc& g, int transA, int transB, hipStream_t s);
-int gemm_dma_glu(const GemmDesc& g, int transA, int transB, hipStream_t s);
+int gemm_dma_glu(const GemmDesc& g, hipStream_t s);
 // the time (us) gemm_dma_bf16's tiles are expected to take, for a choice between the kernels
 double gemm_stream_us(const GemmDesc& g);
 // fp32 C of an unbiased weight gradient (transA, plain epilogue) on streamed tiles, where it wins

@@ -1,6 +1,6 @@
 // gn_gemm_dma.hip — dispatch of the LDS-DMA GEMM core (gn_gemm_dma_core.h) and the VSA
-// unpack-project weight-gradient launch.  The GEMM launches themselves are instantiated in
-// gn_gemm_dma_{f32a,f32b,bf16,glu}.hip.
+// unpack-project weight-gradient launch.  The core's launches are instantiated in
+// gn_gemm_dma_{f32a,f32b,glu}.hip; bf16 outputs take streamed tiles (gn_gemm_stream.hip).
 #include "gn_gemm_dma_core.h"
 
 namespace gn {
@@ -68,9 +68,13 @@ void launch_split_reduce(const GemmDesc& g, hipStream_t s) {
 }
 
 int gemm_dma_launch(const GemmDesc& g, int transA, int transB, int c_dtype, hipStream_t s) {
+    if (g.epi == 1 && (transA || transB)) {
+        set_error("gemm: the GLU epilogue takes untransposed operands only");
+        return GN_E_INVALID;
+    }
     const int wave = gemm_wave_shape(g, transA, transB, c_dtype);
     if (wave >= 0) return gemm_wave_launch(g, wave, transA, transB, c_dtype, s);
-    if (g.epi == 1) return gemm_dma_glu(g, transA, transB, s);
+    if (g.epi == 1) return gemm_dma_glu(g, s);
     if (c_dtype == GN_F32 && gemm_stream_f32_wins(g, transA, transB)) return gemm_stream_f32(g, s);
     if (c_dtype == GN_F32) return transA ? gemm_dma_f32_ta1(g, transB, s) : gemm_dma_f32_ta0(g, transB, s);
     return gemm_dma_bf16(g, transA, transB, s);

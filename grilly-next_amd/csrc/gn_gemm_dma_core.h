@@ -1363,13 +1363,5 @@ int launch_shape(const GemmDesc& g0, hipStream_t s) {
     }
 }
 
-template <typename CT, int EPI>
-int launch_trans(const GemmDesc& g, int ta, int tb, hipStream_t s) {
-    if (!ta && !tb) return launch_shape<false, false, CT, EPI>(g, s);
-    if (!ta && tb) return launch_shape<false, true, CT, EPI>(g, s);
-    if (ta && !tb) return launch_shape<true, false, CT, EPI>(g, s);
-    return launch_shape<true, true, CT, EPI>(g, s);
-}
-
 }  // namespace
 }  // namespace gn

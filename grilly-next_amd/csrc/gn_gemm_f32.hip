@@ -42,19 +42,7 @@ constexpr int PITCH = TK;  // bf16 per LDS row of one plane (32 bytes)
 
 __device__ __forceinline__ int swz(int r) { return (r >> 2) & 1; }
 
-typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
-typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
-
-// (a, b) -> their three bf16 pieces as packed pairs (one v_cvt_pk_bf16_f32 per piece; the
-// pieces widen back to fp32 with a shift or a mask)
-__device__ __forceinline__ void split2(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
-    p0 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){a, b}, bf16x2v));
-    const float ra = a - __uint_as_float(p0 << 16), rb = b - __uint_as_float(p0 & 0xffff0000u);
-    p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){ra, rb}, bf16x2v));
-    const float sa = ra - __uint_as_float(p1 << 16), sb = rb - __uint_as_float(p1 & 0xffff0000u);
-    p2 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){sa, sb}, bf16x2v));
-}
 
 // Operand tile of ROWS rows x TK k, three planes (x0, x1, x2) of ROWS * TK bf16 in LDS.
 //   KCONTIG (element (r, k) at P[r * ld + k]): planes are [ROWS][TK] (32-byte rows, the two

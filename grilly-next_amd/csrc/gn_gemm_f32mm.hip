@@ -163,17 +163,6 @@ int launch_seq(const GemmDesc& g, int ta, int tb, hipStream_t s) {
     return GN_OK;
 }
 
-// (a, b) -> their three bf16 pieces as packed pairs, as gn_gemm_f32.hip splits them
-typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
-typedef float f32x2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void split2(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
-    p0 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){a, b}, bf16x2v));
-    const float ra = a - __uint_as_float(p0 << 16), rb = b - __uint_as_float(p0 & 0xffff0000u);
-    p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){ra, rb}, bf16x2v));
-    const float sa = ra - __uint_as_float(p1 << 16), sb = rb - __uint_as_float(p1 & 0xffff0000u);
-    p2 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){sa, sb}, bf16x2v));
-}
-
 // k 8h .. 8h+7 of one operand row's 16-k stage (h = lane / 32); klim a multiple of 4
 template <bool KC>
 __device__ __forceinline__ void load8(const float* __restrict__ P, int ld, int row, int k0, int klim,

@@ -10,6 +10,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
@@ -24,6 +25,16 @@ __device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
 __device__ __forceinline__ void zero16(f32x16_t& a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) a[r] = 0.f;
+}
+
+// (a, b) -> their three bf16 pieces as packed pairs (one v_cvt_pk_bf16_f32 per piece; the
+// pieces widen back to fp32 with a shift or a mask)
+__device__ __forceinline__ void split2(float a, float b, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
+    p0 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){a, b}, bf16x2_t));
+    const float ra = a - __uint_as_float(p0 << 16), rb = b - __uint_as_float(p0 & 0xffff0000u);
+    p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){ra, rb}, bf16x2_t));
+    const float sa = ra - __uint_as_float(p1 << 16), sb = rb - __uint_as_float(p1 & 0xffff0000u);
+    p2 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){sa, sb}, bf16x2_t));
 }
 
 __device__ __forceinline__ bf16x8_t ld_frag16(const bf16_t* p) {

@@ -521,7 +521,7 @@ def test_glu_linear_bf16(gn, kind):
 @pytest.mark.parametrize("kind", ["swiglu_up", "geglu_up", "reglu_up"])
 def test_ffn_down_glu_fused(gn, M, N, H, kind):
     """gn_ffn_down_glu_bwd (GLU epilogue on dA = dY Wd) + gn_glu_proj_bwd against the
-    unfused oracle chain; the shapes exercise the DMA, register-staged and SIMT GEMMs."""
+    unfused oracle chain; the shapes exercise the DMA-fed and the register-staged products."""
     r = rng_(22)
     K = 128
     X = rnd(r.standard_normal((M, K)).astype(np.float32))
