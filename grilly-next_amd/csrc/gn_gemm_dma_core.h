@@ -137,85 +137,6 @@ __device__ __forceinline__ const bf16_t* stage_base(const bf16_t* P, int ld, int
     return KC ? P + (size_t)r0 * ld + k0 : P + (size_t)k0 * ld + r0;
 }
 
-// A product's operands as a producer wave keeps them: read from the kernel's arguments in one go at
-// its start and held in scalar registers from then on (the empty asm keeps the compiler from
-// loading them again where they are used).  Arguments read where they are needed were scalar loads
-// one after the other ahead of the first DMA and, indexed by segment, between every barrier and its
-// DMA, which a grid of few blocks waits for on every k-tile.  Measured (us): 64 x 768 x 3072 on 6
-// streamed tiles 21.1 -> 18.2, 4096 x 768 x 3072 26.1 -> 23.9.
-struct Operands {
-    const bf16_t *A0, *B0, *A1, *B1;
-    int lda0, ldb0, lda1, ldb1, K0, K1, M, N, nseg;
-    __device__ __forceinline__ explicit Operands(const GemmDesc& g)
-        : A0(g.A[0]), B0(g.B[0]), A1(g.A[1]), B1(g.B[1]), lda0(g.lda[0]), ldb0(g.ldb[0]),
-          lda1(g.lda[1]), ldb1(g.ldb[1]), K0(g.Ks[0]), K1(g.Ks[1]), M(g.M), N(g.N), nseg(g.nseg) {
-        asm volatile("" : "+s"(A0), "+s"(B0), "+s"(A1), "+s"(B1), "+s"(lda0), "+s"(ldb0), "+s"(lda1),
-                     "+s"(ldb1), "+s"(K0), "+s"(K1), "+s"(M), "+s"(N), "+s"(nseg));
-    }
-};
-
-// A producer wave's walk over the k-tiles of one output tile after another.
-template <bool TA, bool TB, int BM, int BN, int NW>
-struct KFeed {
-    static constexpr int NDA = BM / (8 * NW), NDB = BN / (8 * NW);  // DMA instructions of a k-tile
-    const Operands o;
-    const int dw;  // the wave's share of a tile's DMA
-    uint32_t voa[NDA], vob[NDB];
-    const bf16_t *sa, *sb;  // the k-tile's origin in each operand
-    int64_t da, db;         // from one k-tile to the next
-    int m0, n0, left;       // left: k from here to the segment's end
-    bool second;            // the segment
-
-    __device__ __forceinline__ KFeed(const GemmDesc& g, int wave) : o(g), dw(wave) {}
-    // to k = k0 of a segment
-    __device__ __forceinline__ void segment(bool s1, int k0) {
-        second = s1;
-        const int lda = s1 ? o.lda1 : o.lda0, ldb = s1 ? o.ldb1 : o.ldb0;
-        left = (s1 ? o.K1 : o.K0) - k0;
-        stage_offsets<BM, !TA, NW>(lda, m0, o.M, dw, voa);
-        stage_offsets<BN, TB, NW>(ldb, n0, o.N, dw, vob);
-        sa = stage_base<!TA>(s1 ? o.A1 : o.A0, lda, m0, k0);
-        sb = stage_base<TB>(s1 ? o.B1 : o.B0, ldb, n0, k0);
-        da = TA ? (int64_t)BK * lda : BK;
-        db = TB ? BK : (int64_t)BK * ldb;
-    }
-    // to k-tile t (over both segments) of output tile (m, n)
-    __device__ __forceinline__ void start(int m, int n, int t) {
-        m0 = m;
-        n0 = n;
-        const int kt0 = (o.K0 + BK - 1) / BK;
-        segment(t >= kt0, (t < kt0 ? t : t - kt0) * BK);
-    }
-    // The k-tile's DMA; one that its segment's end cuts short (a ragged token count is the K of every
-    // weight gradient) is filled up with zeros.
-    __device__ __forceinline__ void issue(uint32_t base) {
-        constexpr uint32_t B_OFF = BM * BK * 2;
-        if (left >= BK) {
-#pragma unroll
-            for (int q = 0; q < NDA; ++q) dma16s(sa, voa[q], base + 1024u * (uint32_t)(dw * NDA + q));
-#pragma unroll
-            for (int q = 0; q < NDB; ++q) dma16s(sb, vob[q], base + B_OFF + 1024u * (uint32_t)(dw * NDB + q));
-        } else {
-            const int klim = second ? o.K1 : o.K0, k0 = klim - left;
-            stage_tail<BM, !TA, NW>(second ? o.A1 : o.A0, second ? o.lda1 : o.lda0, m0, o.M, k0, klim, dw, base);
-            stage_tail<BN, TB, NW>(second ? o.B1 : o.B0, second ? o.ldb1 : o.ldb0, n0, o.N, k0, klim, dw,
-                                   base + B_OFF);
-        }
-    }
-    // On to the next k-tile; false (and no move) after the product's last.
-    __device__ __forceinline__ bool step() {
-        if (left > BK) {
-            left -= BK;
-            sa += da;
-            sb += db;
-            return true;
-        }
-        if (second || o.nseg < 2) return false;
-        segment(true, 0);
-        return true;
-    }
-};
-
 // A-type fragment (32 rows x 16 k) for v_mfma_f32_32x32x16_bf16: lane l -> row l%32,
 // k = 8(l/32) .. +7 within k-step ks.
 template <int R, bool KC>
@@ -590,9 +511,7 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& g) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
     const int wm = wave >> 1, wn = wave & 1;
     const int dw = wave & 3;  // the wave's slice of a tile's DMA (producer or compute wave)
-    // the compute waves issue the DMA themselves, spread over their MFMAs: whole k-tiles only
-    // (gemm_dma_applicable, choose_tile)
-    constexpr bool SELF_DMA = PROD == 0;
+    constexpr bool SELF_DMA = PROD == 0;  // the compute waves issue the DMA themselves
 
     f32x16_t acc[FM][FN];
 #pragma unroll
@@ -606,11 +525,8 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& g) {
     const int KTall = kt0 + (g.nseg > 1 ? (g.Ks[1] + BK - 1) / BK : 0);
     // split y takes the k-tiles [y KTall / ksplit, (y + 1) KTall / ksplit)
     const int nsplit = g.ksplit < 1 ? 1 : g.ksplit;
-    int kt_lo = 0, KT = KTall;
-    if (nsplit > 1) {
-        kt_lo = (int)(((int64_t)blockIdx.y * KTall) / nsplit);
-        KT = (int)(((int64_t)(blockIdx.y + 1) * KTall) / nsplit) - kt_lo;
-    }
+    const int kt_lo = (int)(((int64_t)blockIdx.y * KTall) / nsplit);
+    const int KT = (int)(((int64_t)(blockIdx.y + 1) * KTall) / nsplit) - kt_lo;
     const int last = KT - 1;
     const bf16_t* const A0 = g.A[0];
     const bf16_t* const A1 = g.A[1];
@@ -768,14 +684,36 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& g) {
     auto dma_all = [&](int tl, int buf) {
         static_for<ND>([&](auto D_) { dma_one(D_, tl, buf); });
     };
+    // The whole DMA of a tile.  With producer waves a segment's K may end inside its last tile
+    // (a ragged token count is the K of every weight gradient): that tile's DMA fills the rest
+    // with zeros.  The self-issuing kernels spread a tile's DMA over their MFMAs and take whole
+    // k-tiles only (gemm_dma_applicable, choose_tile).
+    // (A walk with the next k-tile's origin at hand, as gemm_stream's, lets the DMA out in one burst:
+    // no gain over these grids of a block per tile, and with both operands k-contiguous 8192 x 768 x
+    // 10240 124 -> 136 us.)
+    auto dma_tile = [&](int tl, int buf) {
+        if constexpr (!SELF_DMA) {
+            const int tt = kt_lo + tl;
+            const bool s1 = tt >= kt0;
+            const int k0 = (s1 ? tt - kt0 : tt) * BK, klim = s1 ? g.Ks[1] : g.Ks[0];
+            if (k0 + BK > klim) {
+                const uint32_t base = lds0 + (uint32_t)(buf * STAGE_B);
+                stage_tail<BM, !TA, NW>(s1 ? A1 : A0, s1 ? lda1 : lda0, m0, g.M, k0, klim, dw, base);
+                stage_tail<BN, TB, NW>(s1 ? B1 : B0, s1 ? ldb1 : ldb0, n0, g.N, k0, klim, dw,
+                                       base + A_ELEMS * 2);
+                return;
+            }
+        }
+        dma_all(tl, buf);
+    };
     auto prologue_dma = [&]() {  // tiles 0 .. STAGES-1, then wait for tile 0
         set_offsets(kt_lo >= kt0 ? 1 : 0);
-        dma_all(0, 0);
+        dma_tile(0, 0);
         offsets_for(min(1, last));
-        dma_all(min(1, last), 1);
+        dma_tile(min(1, last), 1);
         if constexpr (STAGES == 3) {
             offsets_for(min(2, last));
-            dma_all(min(2, last), 2);
+            dma_tile(min(2, last), 2);
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * ND));
         } else {
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(ND));
@@ -784,30 +722,18 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& g) {
 
     if constexpr (PROD > 0) {
         if (wave >= 4) {  // producer: the compute waves' barriers, each with the DMA around it
-            // tile i's DMA in order of i; past the last one, the last again
-            KFeed<TA, TB, BM, BN, NW> feed(g, dw);
-            feed.start(m0, n0, kt_lo);
-            int ahead = last;  // k-tiles after the one at feed
-            auto next = [&](int buf) __attribute__((always_inline)) {
-                feed.issue(lds0 + (uint32_t)(buf * STAGE_B));
-                if (ahead > 0) {
-                    --ahead;
-                    feed.step();
-                }
-            };
             if (KT > 0) {
-                static_for<STAGES>([&](auto S_) { next(decltype(S_)::value); });
-                __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 1) * ND));
+                prologue_dma();
                 __syncthreads();
             }
-            int buf = 0;
             for (int t = 0; t < KT; ++t) {
                 // tile t+1 has landed before the barrier that publishes it (tile t+2 may still
                 // be in flight with three stages); tile t's stage is free after it
-                __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 2) * ND));
+                if constexpr (STAGES == 3) __builtin_amdgcn_s_waitcnt(vmcnt_imm(ND));
+                else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
                 __syncthreads();
-                next(buf);
-                buf = buf == STAGES - 1 ? 0 : buf + 1;
+                offsets_for(min(t + STAGES, last));
+                dma_tile(min(t + STAGES, last), t % STAGES);
             }
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
             __syncthreads();
@@ -1270,7 +1196,7 @@ inline TileChoice choose_tile(const GemmDesc& g, bool ta, size_t c_bytes, int ep
     // eager, 8.16 -> 8.09 ms replayed, against the model's 256 x 128.  Shorter k loops keep
     // the model's choice.
     if (epi == 1 && KT >= 12) return {3, 1};
-    // 256 x 256 tiles issue their own DMA and take whole k-tiles only (gemm_body, SELF_DMA)
+    // 256 x 256 tiles issue their own DMA and take whole k-tiles only (gemm_body, dma_tile)
     const int first = k_ragged(g) ? 1 : 0;
     TileChoice best{1, 1};
     double bt = tile_cost(g, ta, c_bytes, epi, 1, 1);
