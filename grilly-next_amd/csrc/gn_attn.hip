@@ -667,6 +667,12 @@ __device__ __forceinline__ float half_max(float v) {
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+// sum over a lane and lane ^ 32
+__device__ __forceinline__ float half_sum(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // Forward producing the backward's saved tensors: O and the fp32 row logsumexp (natural
 // log, S scaled), flash-attention2-rope.glsl:165-247 semantics with the causal mask.  One
 // block per (b*h, 128 queries), four waves x 32 queries; K and V tiles of 64 keys arrive by
@@ -681,9 +687,9 @@ __device__ __forceinline__ float half_max(float v) {
 // bf16 rows; LSE = (m + log2 l) ln 2.
 // Bound by each wave's chain per tile (LDS reads, MFMAs, exponentials, DMA and barrier) more than
 // by any one unit.  Measured (us, replayed): four fragments in flight instead of one, O rescaled only
-// where a maximum moved, the scale inside the exponent's FMA and no mask code without a mask (KB)
-// B4 H16 S2048 D128 causal 106 -> 87, B8 H12 S1024 D64 37 -> 27; S = 1000 (whose last rows sent every
-// tile of their wave down the masked path) 42 -> 27; with a padding mask 56 -> 30.
+// where a maximum moved, the masked entries' code on the tiles that have some and no key-mask code
+// without a mask (KB) B4 H16 S2048 D128 causal 105 -> 88, B8 H12 S1024 D64 38 -> 27; S = 1000 (whose
+// last rows sent every tile of their wave down the masked path) 43 -> 27; with a padding mask 55 -> 33.
 template <int D, bool KB>
 __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc tV, TDesc tO,
                                                      float* __restrict__ LSE,
@@ -775,15 +781,17 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
         for (int j = 0; j < RING; ++j) fv[j] = frag_cols<D>(sV, 16 * (j / NT), 32 * (j % NT));
         __builtin_amdgcn_sched_barrier(0);
 
-        // scores to base-2 units, masked entries to -inf (P = 0), on the tiles that need it; the
-        // others keep the raw products and scale inside the exponent's FMA
-        const bool raw = full && !biased && c2 > 0.f;
-        if (!raw) {
+        // scores in base-2 units; masked entries, on the tiles that have some, are -inf (P = 0)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[i][r] *= c2;
+        if (!full || biased) {
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    float v = sc[i][r] * c2;
+                    float v = sc[i][r];
                     if (biased) v += __shfl(kbl, 32 * i + 8 * (r >> 2) + 4 * h + (r & 3));
                     if (!full) v = 32 * i + 8 * (r >> 2) + (r & 3) <= klim ? v : -INFINITY;
                     sc[i][r] = v;
@@ -792,11 +800,12 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
         float mt = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 16; ++r) mt = fmaxf(mt, fmaxf(sc[0][r], sc[1][r]));
-        const float f = raw ? c2 : 1.0f;
         // The maximum is the row's own after every tile, so that a row's leading weight is exactly 1
-        // in bf16: one that lags behind (O and l then rescaled on few tiles) rounds every weight of
-        // the row, and the errors of the leading ones do not average out.
-        const float mn = fmaxf(m, half_max(mt) * f);
+        // in bf16: one that lags behind (O and l then rescaled on few tiles)
+        // rounds every weight of the row, and the errors of the leading ones do not average out.  The
+        // scale's own rounding and one chain of a tile's sum keep the results' bits; inside the exponent's
+        // FMA and in four chains they would be 0 to 3 % faster.
+        const float mn = fmaxf(m, half_max(mt));
         const float ms = mn == -INFINITY ? 0.f : mn;  // a row with no visible key yet stays empty
         const float alpha = __builtin_amdgcn_exp2f(m - ms);
         if (__any(mn > m)) {
@@ -806,19 +815,19 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
                 for (int r = 0; r < 16; ++r) aO[t][r] *= alpha;
         }
         m = mn;
-        float ps[4];  // the tile's sum in four chains, then onto the row's
+        float ps = 0.f;
         bf16x8_t pb[4];
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             float pv[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                pv[e] = __builtin_amdgcn_exp2f(fmaf(sc[p >> 1][8 * (p & 1) + e], f, -ms));
-                ps[p] = e == 0 ? pv[0] : ps[p] + pv[e];
+                pv[e] = __builtin_amdgcn_exp2f(sc[p >> 1][8 * (p & 1) + e] - ms);
+                ps += pv[e];
             }
             pb[p] = to_bf16x8(pv[0], pv[1], pv[2], pv[3], pv[4], pv[5], pv[6], pv[7]);
         }
-        l = l * alpha + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
+        l = l * alpha + half_sum(ps);  // with the other 16 keys of every 32
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < 4 * NT; ++j) {
@@ -828,7 +837,6 @@ __global__ __launch_bounds__(256) void attn_fwd_mfma(TDesc tQ, TDesc tK, TDesc t
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    l += __shfl_xor(l, 32);  // the other 16 keys of every 32
 
     __syncthreads();
     float* st = reinterpret_cast<float*>(smem) + wave * 32 * (D + 4);
