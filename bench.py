@@ -81,12 +81,11 @@ def parse():
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "ffn_dominant_gemm_hbm_traffic.txt")
 # The launches of the FFN step's two largest calls as rocprof names them: (kernel pattern,
-# work-items per dispatch).  [dWg;dWu] (transposed A, fp32 C) and dN run one launch each on
-# 256 x 128 tiles with three LDS stages and four producer waves (512 threads per block):
-# 704 and 256 blocks.
+# work-items per dispatch).  [dWg;dWu] (transposed A, fp32 C) and dN run one launch each of
+# 512-thread blocks, one per CU, over 704 and 256 streamed 256 x 128 tiles.
 CALL_KERNELS = {
-    "[dWg;dWu]": [(r"gemm_core<true, false, float, 256, 128, 0, 3, false, 4>", 704 * 512)],
-    "dN": [(r"gemm_core<false, false, unsigned short, 256, 128, 0, 3, false, 4>", 256 * 512)],
+    "[dWg;dWu]": [(r"gemm_stream<true, false, float, 256, 128, 3>", 256 * 512)],
+    "dN": [(r"gemm_stream<false, false, unsigned short, 256, 128, 3>", 256 * 512)],
 }
 DOMINANT_CALL = "[dWg;dWu]"
 CALIB_FLOATS = 1 << 28

@@ -7,7 +7,8 @@
 // producer waves run on into the next tile's k-tiles while the four compute waves store the
 // finished one, and the store goes out through 4 KB of LDS per wave, so that a tile costs
 // its k-tiles and ~3 us.  What bounds it: at 12 k-tiles the store bursts and the k-tiles about
-// equally, from ~32 k-tiles on the matrix cores and the LDS reads that feed them.
+// equally, from ~32 k-tiles on the matrix cores (63-68 % busy over 4096 x 2048 x 11264 and dW 11264 x
+// 2048 x 4096) and the LDS reads that feed them.
 //   us, a block per tile -> here (A k-contiguous, B row-major [N][K]; in brackets B [K][N]):
 //   8192 x 32000 x 768  689 -> 447 (668 -> 464)    8192 x 3072 x 768   63 -> 42
 //   2001 x 32000 x 768  152 -> 99                  8192 x  768 x 768   19 -> 15 (16 -> 14)
