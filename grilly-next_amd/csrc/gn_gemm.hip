@@ -564,8 +564,9 @@ int colsum_dispatch(const void* in, float* out, int M, int N, int dtype, unsigne
 // pitch ldx), rows of dW below Msplit to dW, the rest to dW2 (row - Msplit), and the bias
 // gradient db = column sums of dY (db for rows < Msplit, db2 beyond) when db != nullptr.
 // The bias rides on the GEMM (row sums of its A fragments) when the LDS-DMA core takes the
-// shape; otherwise a two-pass column sum runs first, staged in dW (which the GEMM then
-// overwrites) unless accumulating.
+// shape (and is not better off without: gemm_stream_sums_apart); otherwise a column sum runs
+// first, of more than 1024 rows in two passes staged in dW (which the GEMM then overwrites) unless
+// accumulating.
 int weight_grad(const void* dY, int ldy, const void* X, int ldx, int M, int N, int Kin, void* dW,
                 void* dW2, int Msplit, float* db, float* db2, int dtype, unsigned flags,
                 hipStream_t s, void* ws = nullptr, size_t ws_bytes = 0, bool beside = false) {
