@@ -116,7 +116,7 @@ __global__ __launch_bounds__(512, 1) void gemm_stream(GemmDesc g) {
     const int nblk = tilesM * tilesN;
     const int ntile = (nblk - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;  // this block's
     // its i-th tile: block b runs on XCD b % 8, each XCD walks one contiguous range of the tiles,
-    // GROUP tile rows at a time (gridDim.x is a multiple of 8, or the tiles are one round)
+    // GROUP tile rows at a time (gridDim.x is a multiple of 8, or a block has one tile)
     auto tile_at = [&](int i, int& m0, int& n0) __attribute__((always_inline)) {
         const int x = (int)blockIdx.x + i * (int)gridDim.x;
         const int xcd = x & 7, per = nblk >> 3, extra = nblk & 7;
